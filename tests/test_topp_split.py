@@ -1,0 +1,104 @@
+"""Top-p rows over several workgroups (rows longer than one workgroup's
+registers): ragged and padded lengths, both element types, penalties, masks,
+greedy and invalid rows, ties past the ranked capacity, top-p off and near
+zero, infinities and NaN; bit-exact against the oracle.  On the CPU every
+workgroup of the launch runs at once (the exchange) or one after another
+(every poll runs out: the fallbacks)."""
+import os
+import shutil
+import sys
+
+import numpy as np
+import pytest
+
+import gpu_harness as H
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.abspath(__file__)), "cpu_sim"))
+
+
+def _rows(oracle, V, seed, bf16=False, mask=False, hist=64):
+    """One row of each kind the kernel tells apart."""
+    from tinygpt_amd import workloads as W
+
+    g = np.random.default_rng(seed)
+    kinds = ["plain", "flat", "greedy", "special", "coarse", "inf", "none", "invalid"]
+    B = len(kinds)
+    x = (g.standard_normal((B, V)) * 3.0).astype(np.float32)
+    p = oracle.make_params(B, temperature=0.8, top_k=0, top_p=0.9, repetition=1.1, presence=0.2, frequency=0.1)
+    p["temperature"][3], p["temperature"][4] = 1.0, 0.5
+    p["top_p"][[3, 4]] = [1.0, 1e-9]
+    p["top_k"][[0, 3]] = [-1, V + 3]
+    x[1] = 0.75  # every id in one bucket, more than the lists and the ranking hold
+    x[1, ::3] = 0.7
+    p["temperature"][2] = 0.0
+    x[3, g.choice(V, V // 20, replace=False)] = np.nan
+    x[3, g.choice(V, V // 20, replace=False)] = -np.inf
+    x[4] = np.round(x[4])
+    x[5, [5, V - 1]] = np.inf
+    x[6] = -np.inf
+    p["temperature"][7] = np.nan
+    table = None
+    if mask:
+        words = (V + 31) // 32
+        table = g.integers(0, 1 << 32, (3, words), dtype=np.uint64).astype(np.uint32)
+        table[1] = 0
+        table[1, [0, words // 2, words - 1]] = 1
+        table[:, -1] &= np.uint32((1 << (V - 32 * (words - 1))) - 1) if V % 32 else np.uint32(0xFFFFFFFF)
+        p["mask_state"] = [0, 1, 2, -1, 0, 1, 2, 0]
+    h = g.integers(-2, V + 2, (B, hist)).astype(np.int32) if hist else None
+    hl = g.integers(0, hist + 1, B).astype(np.int32) if hist else None
+    u = (g.integers(0, 1 << 24, B) / (1 << 24)).astype(np.float32)
+    return (W.f32_to_bf16_bits(x) if bf16 else x), p, u, h, hl, table
+
+
+def _oracle(oracle, x, p, u, h, hl, table):
+    return oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=8, want_post=True, nthreads=8)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("rows,V,bf16,mask,concurrent", [
+    ([0, 1], 32769, False, False, True), ([2, 3], 33001, True, True, True), ([4, 5], 36864, False, True, True),
+    ([6, 7], 32800, True, False, True), ([0, 1, 2, 4], 33003, True, False, False), ([3, 5], 33002, False, True, False)])
+def test_split_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
+    import sim as S
+
+    import tinygpt_amd as tg
+
+    S.build()
+    x, p, u, h, hl, table = _rows(oracle, V, 7 + V, bf16, mask)
+    x, p, u, h, hl = x[rows], p[rows], u[rows], h[rows], hl[rows]
+    hint = tg.batch_hint(p, V)
+    r = S.run_sample(x, p, u, h, hl, mask_table=table, kept_cap=8, hint=hint, concurrent=concurrent,
+                     repeat=2 if concurrent else 1, env_extra={"TGS_KEY_SPINS": "100000"} if concurrent else None)
+    assert all(blk == 512 and grid > len(rows) for grid, blk in r["launches"])
+    H.compare(r, _oracle(oracle, x, p, u, h, hl, table), p, V, what="split top-p")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,bf16,mask,hist", [
+    (32769, False, False, 64), (32776, True, True, 64), (50001, True, False, 0), (65536, False, True, 1000),
+    (128256, False, False, 64), (128256, True, True, 0), (151936, True, False, 256), (151935, False, True, 64)])
+def test_split_rows(sampler, oracle, V, bf16, mask, hist):
+    x, p, u, h, hl, table = _rows(oracle, V, V, bf16, mask, hist)
+    o = _oracle(oracle, x, p, u, h, hl, table)
+    for hint in ("auto", None):  # the launch alone, and behind the general kernels
+        H.log(f"case split top-p V={V} bf16={bf16} mask={mask} hint={hint}")
+        r = H.run_gpu(sampler, x, p, u, h, hl, mask_table=table, kept_cap=8, hint=hint)
+        H.compare(r, o, p, V, what="split top-p")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [1, 3, 33, 200])
+def test_split_batches(sampler, oracle, B):
+    """Chunk counts from the most to the fewest, and a batch over several
+    launches (its slabs outnumber the workspace's)."""
+    V = 128256
+    g = np.random.default_rng(B)
+    x = (g.standard_normal((B, V)) * 3.0).astype(np.float32)
+    p = oracle.make_params(B, temperature=g.choice([0.7, 1.0, 1.3], B), top_k=0, top_p=g.choice([0.3, 0.9, 1.0], B))
+    u = (g.integers(0, 1 << 24, B) / (1 << 24)).astype(np.float32)
+    o = _oracle(oracle, x, p, u, None, None, None)
+    for _ in range(2):
+        H.log(f"case split top-p batch B={B}")
+        r = H.run_gpu(sampler, x, p, u, kept_cap=8, hint="auto")
+        H.compare(r, o, p, V, what="split top-p")

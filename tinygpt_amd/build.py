@@ -19,7 +19,7 @@ OUT = os.path.join(HERE, "libtgs_sampler.so")
 # its own library: not part of the sampler's C ABI)
 FLOOR_SRC = "tgs_floor.hip"
 FLOOR_OUT = os.path.join(HERE, "libtgs_floor.so")
-SOURCES = ["tgs_kernels.hip", "tgs_k64.hip", "tgs_spec.hip", "tgs_topp.hip", "tgs_topk.hip", "tgs_logprob.hip",
+SOURCES = ["tgs_kernels.hip", "tgs_k64.hip", "tgs_spec.hip", "tgs_topp.hip", "tgs_topp_split.hip", "tgs_topk.hip", "tgs_logprob.hip",
            "tgs_mask.hip", "tgs_api.hip"]
 ARCH = os.environ.get("TGS_OFFLOAD_ARCH", "gfx950")
 

@@ -30,9 +30,12 @@ struct tgs_ctx {
   unsigned long long* ws = nullptr;
   int* ws_cnt = nullptr;
   int ws_rows = 0;  // chunk lists of KMAX entries the workspace holds
-  unsigned* k64_cnt = nullptr;  // fused kernel exchange lines (arrival counter, epoch, count words), one per row
+  size_t ws_words = 0;  // its 8-byte words
+  // one allocation, zeroed once, from k64_lists on
   unsigned long long* k64_lists = nullptr;  // fused kernel chunk lists, [max_batch * kMaxSplit][64]
   unsigned long long* k64_keys = nullptr;   // fused kernel bound-exchange keys, [max_batch][K64_KEYS]
+  unsigned long long* tp_lines = nullptr;   // split top-p exchange lines, [max_batch][TOPPS_LINE]
+  unsigned* k64_cnt = nullptr;  // fused kernel exchange lines (arrival counter, epoch, count words), one per row
   uint32_t* mask_table = nullptr;
   int n_states = 0, mask_vocab = 0, mask_words = 0;
   void* mask_stage = nullptr;  // tgs_mask_table_update staging (grown on demand)
@@ -132,6 +135,16 @@ int choose_split(int num_cu, int ws_rows, int B, int V) {
   return S;
 }
 
+// Chunks per row of the split top-p kernel: about one workgroup per CU, at
+// least what its registers need, chunks of at least 4096 ids (below that the
+// row's exchanges outweigh the work a further chunk takes over), in slabs the
+// workspace holds.
+int choose_split_topp(int num_cu, int B, int V) {
+  const int smin = (V + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
+  const int S = std::min({tgs::TOPPS_MAX_SPLIT, num_cu / std::max(B, 1), V / 4096});
+  return std::max(S, smin);
+}
+
 // Static LDS of the fused kernel beyond its dynamic carve-up (wave lists,
 // staging, the radix-select scratch and the merge's words), with room for
 // alignment.
@@ -175,6 +188,8 @@ struct SampleRes {
   unsigned long long* ws = nullptr;  // [ws_rows][KMAX] general-path chunk lists
   int* ws_cnt = nullptr;             // [ws_rows * (KMAX / 64)]
   int ws_rows = 0;
+  size_t ws_words = 0;                      // ws in 8-byte words (split top-p slabs)
+  unsigned long long* tp_lines = nullptr;   // [rows * TOPPS_LINE], zeroed at set-up
   unsigned* k64_cnt = nullptr;              // [rows * K64_CNT_STRIDE], zeroed at set-up
   unsigned long long* k64_lists = nullptr;  // [rows * kMaxSplit][64], entries 0 between calls
   unsigned long long* k64_keys = nullptr;   // [rows * K64_KEYS], zeroed at set-up
@@ -185,6 +200,34 @@ struct SampleRes {
 int efail(std::string& err, int code, const std::string& msg) {
   err = msg;
   return code;
+}
+
+// The rows without a top-k (all of a batch's, greedy rows too, with
+// a.topp_all): one workgroup per row where a row fits its registers, several
+// per row beyond.
+int topp_core(const SampleRes& res, std::string& err, tgs::SampleArgs a, tgs_dtype dt, hipStream_t stream) {
+  hipError_t e;
+  if (a.V > tgs::topp_resident_ids()) {
+    const int S = choose_split_topp(res.num_cu, a.B, a.V);
+    const int rows = (int)(res.ws_words / tgs::TOPPS_PAIR / (size_t)S);
+    if (rows < 1) return efail(err, TGS_ETOOBIG, "workspace too small for top-p rows");
+    a.L = ((a.V + S - 1) / S + 63) / 64 * 64;
+    a.S = (a.V + a.L - 1) / a.L;
+    a.ws = res.ws;
+    a.tp_lines = res.tp_lines;
+    // polls of a row's maxima and of its decision before a workgroup goes on
+    // without its partners (TGS_KEY_SPINS overrides: tests)
+    const char* env = std::getenv("TGS_KEY_SPINS");
+    a.key_spins = env ? std::max(0, std::atoi(env)) : 1024;
+    e = tgs::launch_topps(a, dt, rows, stream);
+  } else {
+    a.S = 1;
+    a.L = a.V;
+    a.topp_cap = tgs::topp_pack_cap(a.V, a.TS, res.lds_limit - 2 * sizeof(tgs::BlockScratch));
+    e = tgs::launch_topp(a, dt, stream);
+  }
+  if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
+  return TGS_OK;
 }
 
 // Validates the call and launches the kernels the batch hint selects (the
@@ -307,15 +350,10 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
   const int mink = hint ? hint->min_top_k : 0;
   if (mk >= V && mink >= V && tgs::topp_lds_bytes(V, a.TS) + 2 * sizeof(tgs::BlockScratch) <= res.lds_limit) {
     // every sampling row without a usable top-k: the top-p kernel serves the
-    // batch alone, greedy rows included (one workgroup per row)
+    // batch alone, greedy rows included
     a.full_rows = 1;
     a.topp_all = 1;
-    a.S = 1;
-    a.L = V;
-    a.topp_cap = tgs::topp_pack_cap(V, a.TS, res.lds_limit - 2 * sizeof(tgs::BlockScratch));
-    hipError_t e = tgs::launch_topp(a, dt, stream);
-    if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
-    return TGS_OK;
+    return topp_core(res, err, a, dt, stream);
   }
   a.full_rows = (mk > tgs::KMAX || mk >= V) ? 1 : 0;
   const int S = choose_split(res.num_cu, res.ws_rows, B, V);
@@ -333,10 +371,9 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS");
   if (a.full_rows && tgs::topp_lds_bytes(V, a.TS) + 2 * sizeof(tgs::BlockScratch) > res.lds_limit)
     return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS (top-p rows)");
-  a.topp_cap = tgs::topp_pack_cap(V, a.TS, res.lds_limit - 2 * sizeof(tgs::BlockScratch));
   hipError_t e = tgs::launch_sample(a, dt, lds, stream);
   if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
-  return TGS_OK;
+  return a.full_rows ? topp_core(res, err, a, dt, stream) : TGS_OK;
 }
 
 // ---------------------------------------------------------------- allocation-free sampling
@@ -347,6 +384,7 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
 //   [k64 chunk lists: kNaRows * kMaxSplit * 64 u64, entries 0 between calls]
 //   [k64 bound-exchange keys: kNaRows * K64_KEYS u64]
 //   [general-path chunk lists: kNaWsRows * KMAX u64]
+//   [split top-p exchange lines: kNaRows * TOPPS_LINE u64]
 //   [k64 exchange lines: kNaRows * K64_CNT_STRIDE u32, counters zero between calls]
 //   [general-path list counts: kNaWsRows * (KMAX / 64) i32]
 // The k64 kernel leaves its lists and counters in that state after every
@@ -360,9 +398,10 @@ constexpr int kNaHist = tgs::K64_MAX_HIST;
 constexpr size_t kNaListWords = (size_t)kNaRows * kMaxSplitK64 * 64;
 constexpr size_t kNaKeyWords = (size_t)kNaRows * tgs::K64_KEYS;
 constexpr size_t kNaWsWords = (size_t)kNaWsRows * tgs::KMAX;
+constexpr size_t kNaTpWords = (size_t)kNaRows * tgs::TOPPS_LINE;
 constexpr size_t kNaCntU32 = (size_t)kNaRows * tgs::K64_CNT_STRIDE;
 constexpr size_t kNaWsCntI32 = (size_t)kNaWsRows * (tgs::KMAX / 64);
-constexpr size_t kNaWords = kNaListWords + kNaKeyWords + kNaWsWords + (kNaCntU32 + kNaWsCntI32) / 2;
+constexpr size_t kNaWords = kNaListWords + kNaKeyWords + kNaWsWords + kNaTpWords + (kNaCntU32 + kNaWsCntI32) / 2;
 static_assert(kNaCntU32 % 2 == 0 && kNaWsCntI32 % 2 == 0, "whole 8-byte words");
 
 constexpr int kNaMaxDevices = 64;
@@ -411,6 +450,7 @@ int noalloc_setup(int device, NoAllocDevice*& out) {
     if (tgs::set_sample_lds_limit(d.lds_limit - sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_k64_lds_limit(d.lds_limit - k64_static()) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_topp_lds_limit(d.lds_limit - 2 * sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
+    if (tgs::set_topps_lds_limit(d.lds_limit - tgs::topps_static_lds() - 256) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_topk_lds_limit(d.lds_limit - 2 * sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
     // everything zero: k64 lists "not written", counters and epochs zero
     hipLaunchKernelGGL(na_fill_kernel, dim3(1024), dim3(256), 0, nullptr, d.ptr, kNaWords);
@@ -482,17 +522,25 @@ int tgs_create(tgs_handle* out, int device, int max_batch, int max_vocab, int ma
   if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && v > 0)
     h->lds_limit = (size_t)v;
   h->ws_rows = std::max(max_batch, 4 * h->num_cu);
-  hipError_t e = hipMalloc(&h->ws, sizeof(unsigned long long) * (size_t)h->ws_rows * tgs::KMAX);
+  // (and room for the split top-p kernel's slabs of 1024 chunks at a time)
+  h->ws_words = std::max((size_t)h->ws_rows * tgs::KMAX,
+                         max_vocab > tgs::topp_resident_ids()
+                             ? (size_t)std::min(1024, max_batch * tgs::TOPPS_MAX_SPLIT) * tgs::TOPPS_PAIR
+                             : (size_t)0);
+  hipError_t e = hipMalloc(&h->ws, sizeof(unsigned long long) * h->ws_words);
   if (e == hipSuccess) e = hipMalloc(&h->ws_cnt, sizeof(int) * (size_t)h->ws_rows * (tgs::KMAX / 64));
-  const size_t cnt_bytes = sizeof(unsigned) * (size_t)max_batch * tgs::K64_CNT_STRIDE;
-  if (e == hipSuccess) e = hipMalloc(&h->k64_cnt, cnt_bytes);
-  if (e == hipSuccess) e = hipMemset(h->k64_cnt, 0, cnt_bytes);
-  const size_t list_bytes = sizeof(unsigned long long) * (size_t)max_batch * kMaxSplit * 64;
-  if (e == hipSuccess) e = hipMalloc(&h->k64_lists, list_bytes);
-  if (e == hipSuccess) e = hipMemset(h->k64_lists, 0, list_bytes);  // every entry "not written"
-  const size_t key_bytes = sizeof(unsigned long long) * (size_t)max_batch * tgs::K64_KEYS;
-  if (e == hipSuccess) e = hipMalloc(&h->k64_keys, key_bytes);
-  if (e == hipSuccess) e = hipMemset(h->k64_keys, 0, key_bytes);
+  // everything that starts zeroed in one allocation: chunk lists ("not
+  // written"), keys, exchange lines, counters and epochs
+  const size_t rows = (size_t)max_batch;
+  const size_t n_lists = rows * kMaxSplit * 64, n_keys = rows * tgs::K64_KEYS, n_tp = rows * tgs::TOPPS_LINE;
+  const size_t zero_bytes = sizeof(unsigned long long) * (n_lists + n_keys + n_tp) + sizeof(unsigned) * rows * tgs::K64_CNT_STRIDE;
+  if (e == hipSuccess) e = hipMalloc(&h->k64_lists, zero_bytes);
+  if (e == hipSuccess) e = hipMemset(h->k64_lists, 0, zero_bytes);
+  if (e == hipSuccess) {
+    h->k64_keys = h->k64_lists + n_lists;
+    h->tp_lines = h->k64_keys + n_keys;
+    h->k64_cnt = (unsigned*)(h->tp_lines + n_tp);
+  }
   if (e == hipSuccess) {
     // raise the dynamic-LDS ceiling to the device limit; a runtime that
     // rejects the attribute keeps its default (calls that need more fail
@@ -500,6 +548,7 @@ int tgs_create(tgs_handle* out, int device, int max_batch, int max_vocab, int ma
     if (tgs::set_sample_lds_limit(h->lds_limit - sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_k64_lds_limit(h->lds_limit - k64_static()) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_topp_lds_limit(h->lds_limit - 2 * sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
+    if (tgs::set_topps_lds_limit(h->lds_limit - tgs::topps_static_lds() - 256) != hipSuccess) (void)hipGetLastError();
     if (tgs::set_topk_lds_limit(h->lds_limit - 2 * sizeof(tgs::BlockScratch)) != hipSuccess) (void)hipGetLastError();
     e = hipDeviceSynchronize();
   }
@@ -516,9 +565,7 @@ void tgs_destroy(tgs_handle h) {
   DeviceGuard g(h->device);
   if (h->ws) (void)hipFree(h->ws);
   if (h->ws_cnt) (void)hipFree(h->ws_cnt);
-  if (h->k64_cnt) (void)hipFree(h->k64_cnt);
   if (h->k64_lists) (void)hipFree(h->k64_lists);
-  if (h->k64_keys) (void)hipFree(h->k64_keys);
   if (h->mask_table) (void)hipFree(h->mask_table);
   if (h->mask_stage) (void)hipFree(h->mask_stage);
   free_spec(h);
@@ -645,6 +692,8 @@ int tgs_sample(tgs_handle h, const void* d_logits, tgs_dtype dt, int B, int V, i
   res.ws = h->ws;
   res.ws_cnt = h->ws_cnt;
   res.ws_rows = h->ws_rows;
+  res.ws_words = h->ws_words;
+  res.tp_lines = h->tp_lines;
   res.k64_cnt = h->k64_cnt;
   res.k64_lists = h->k64_lists;
   res.k64_keys = h->k64_keys;
@@ -693,7 +742,9 @@ int tgs_sample_noalloc(int device, const void* d_logits, tgs_dtype dt, int B, in
   res.k64_keys = d->ptr + kNaListWords;
   res.ws = d->ptr + kNaListWords + kNaKeyWords;
   res.ws_rows = kNaWsRows;
-  res.k64_cnt = (unsigned*)(d->ptr + kNaListWords + kNaKeyWords + kNaWsWords);
+  res.ws_words = kNaWsWords;
+  res.tp_lines = d->ptr + kNaListWords + kNaKeyWords + kNaWsWords;
+  res.k64_cnt = (unsigned*)(res.tp_lines + kNaTpWords);
   res.ws_cnt = (int*)(res.k64_cnt + kNaCntU32);
   res.mask_table = n_states > 0 ? d_mask_table : nullptr;
   res.n_states = n_states;

@@ -1,6 +1,6 @@
 // tgs_bucket.h -- the count and exact-mass histogram over buckets below the
 // row maximum that the top-k and top-p kernels place their cut and draw
-// with (one workgroup of 1024 threads per row).
+// with.
 //
 // A composite with canonical logit y under the row maximum m lands in
 // bucket floor((m - y) * 32) (0 at y == m); y - m <= -32 (mass 0) lands in

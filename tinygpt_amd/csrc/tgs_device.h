@@ -448,6 +448,47 @@ __device__ __forceinline__ K block_select_kth(Enum en, unsigned kth, BlockScratc
   return prefix;
 }
 
+// One digit of a mass-weighted radix selection, by one wave: the highest
+// digit d of the 256-bin histogram s.hc / s.hm whose inclusive prefix (from
+// the top, on mass_above) reaches target, into s.sel, with the mass and the
+// count ahead of it (s.mass_above, s.cnt_above) and its own count (s.binc_i).
+__device__ __forceinline__ void mass_digit_scan(BlockScratch& s, u64 target, u64 mass_above, unsigned cnt_above) {
+  const int lane = threadIdx.x;
+  unsigned cs[4];
+  u64 ms[4];
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    cs[j] = s.hc[255 - 4 * lane - j];
+    ms[j] = s.hm[255 - 4 * lane - j];
+  }
+  u64 lm = ms[0] + ms[1] + ms[2] + ms[3];
+  unsigned lc = cs[0] + cs[1] + cs[2] + cs[3];
+  u64 cm = wave_incl_scan(lm) - lm + mass_above;
+  unsigned cc = wave_incl_scan(lc) - lc + cnt_above;
+  int found = -1;
+  u64 ab = 0;
+  unsigned ca = 0, bc = 0;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    if (found < 0 && cs[j] > 0 && cm + ms[j] >= target) {
+      found = 255 - 4 * lane - j;
+      ab = cm;
+      ca = cc;
+      bc = cs[j];
+    }
+    cm += ms[j];
+    cc += cs[j];
+  }
+  u64 bal = __ballot(found >= 0);
+  int first = __ffsll((long long)bal) - 1;
+  if (lane == first) {
+    s.sel = found;
+    s.mass_above = ab;
+    s.cnt_above = ca;
+    s.binc_i = (int)bc;
+  }
+}
+
 // Mass-based MSB radix select over unique 64-bit composite keys, each with
 // an integer mass.  Finds the element i (in descending key order) that is
 // the first with C_i >= target, where C_i is the inclusive mass prefix.
@@ -476,42 +517,7 @@ __device__ __forceinline__ u64 block_mass_select(Enum en, u64 target, BlockScrat
       }
     });
     __syncthreads();
-    if (threadIdx.x < 64) {
-      const int lane = threadIdx.x;
-      unsigned cs[4];
-      u64 ms[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        cs[j] = s.hc[255 - 4 * lane - j];
-        ms[j] = s.hm[255 - 4 * lane - j];
-      }
-      u64 lm = ms[0] + ms[1] + ms[2] + ms[3];
-      unsigned lc = cs[0] + cs[1] + cs[2] + cs[3];
-      u64 cm = wave_incl_scan(lm) - lm + mass_above;
-      unsigned cc = wave_incl_scan(lc) - lc + cnt_above;
-      int found = -1;
-      u64 ab = 0;
-      unsigned ca = 0, bc = 0;
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        if (found < 0 && cs[j] > 0 && cm + ms[j] >= target) {
-          found = 255 - 4 * lane - j;
-          ab = cm;
-          ca = cc;
-          bc = cs[j];
-        }
-        cm += ms[j];
-        cc += cs[j];
-      }
-      u64 bal = __ballot(found >= 0);
-      int first = __ffsll((long long)bal) - 1;
-      if (lane == first) {
-        s.sel = found;
-        s.mass_above = ab;
-        s.cnt_above = ca;
-        s.binc_i = (int)bc;
-      }
-    }
+    if (threadIdx.x < 64) mass_digit_scan(s, target, mass_above, cnt_above);
     __syncthreads();
     const int d = s.sel;
     mass_above = s.mass_above;
@@ -739,6 +745,10 @@ __device__ __forceinline__ uint32_t wave_or(uint32_t x) {
   x |= xor_lane32<2>(x);
   x |= xor_lane32<1>(x);
   return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+}
+
+__device__ __forceinline__ u64 wave_or64(u64 x) {
+  return ((u64)wave_or((uint32_t)(x >> 32)) << 32) | wave_or((uint32_t)x);
 }
 
 // Number of set bits of a wave mask below this lane.

@@ -28,10 +28,23 @@ constexpr int K64_CNT_WORDS = 32;
 constexpr int K64_KEYS = 256;
 
 // Top-p kernel (rows without a top-k): threads per workgroup and the most
-// ids of one histogram bucket ranked in LDS.
+// ids of the cut's and the draw's histogram buckets gathered in LDS.
 constexpr int TOPP_NT = 1024;
-constexpr int TOPP_CAP = 1024;
+constexpr int TOPP_CAP = 2816;
 constexpr int TOPP_MASK_PRE = 2;  // register-resident row vectors requested before the mask words
+
+// Split top-p kernel (rows too long for the top-p kernel's registers):
+// threads per workgroup, chunks per row at most, ids per chunk at most, and
+// in 8-byte words: the exchange line of a row, and of a (row, chunk) its
+// slab (NB masses, NB + 1 counts and a pad), one of the two lists behind it
+// (ids of the cut's and the draw's buckets) and all together.
+constexpr int TOPPS_NT = 512;
+constexpr int TOPPS_MAX_SPLIT = 16;
+constexpr int TOPPS_CHUNK = TOPPS_NT * 32;
+constexpr int TOPPS_LINE = 64;
+constexpr int TOPPS_SLAB = 1024 + 514;
+constexpr int TOPPS_LIST = 192;
+constexpr int TOPPS_PAIR = TOPPS_SLAB + 2 * TOPPS_LIST;
 
 // Top-k kernel (1 <= top_k <= KMAX, the row held in registers): threads per
 // workgroup and candidate capacity.
@@ -71,6 +84,8 @@ struct SampleArgs {
   int full_rows;         // 1: full_kernel runs after the chunk kernels
   int hint_k;            // the launch hint's max_top_k (INT_MAX without a hint)
   int topp_all;          // 1: the top-p kernel alone serves the batch (its greedy rows too)
+  unsigned long long* tp_lines;  // split top-p kernel: [rows][TOPPS_LINE] exchange lines (zero at set-up)
+  int row0;              // split top-p kernel: the launch's first row (slabs are indexed from it)
   int topp_cap;          // top-p kernel: allowed ids packed into LDS (beyond topp_lds_bytes)
   tgs_debug dbg;
 };
@@ -154,8 +169,7 @@ constexpr int SPEC_GROUPS = 4;  // 16-byte vector groups per block of 1024 ids (
 
 // Launches the chunk kernel, the merge kernel when rows are split (a.S > 1)
 // and, when a.full_rows is set, the full-path kernel (rows with
-// KMAX < top_k < V) and the top-p kernel (rows without a top-k), in that
-// order on st.
+// KMAX < top_k < V), in that order on st.
 hipError_t launch_sample(const SampleArgs& a, int dtype, size_t lds, hipStream_t st);
 hipError_t set_sample_lds_limit(size_t bytes);
 // The fused kernel for batches of greedy rows and rows with top_k <= 64:
@@ -179,6 +193,13 @@ int topp_pack_cap(int V, int TS, size_t lds_avail);
 // Dynamic LDS: topp_lds_bytes + a.topp_cap packed ids.
 hipError_t launch_topp(const SampleArgs& a, int dtype, hipStream_t st);
 hipError_t set_topp_lds_limit(size_t bytes);
+// Longest row the top-p kernel holds in registers.
+int topp_resident_ids();
+// The same rows over a.S chunks of a.L ids each, `rows` rows per launch
+// (their slabs lie in a.ws); dynamic LDS topp_lds_bytes.
+hipError_t launch_topps(SampleArgs a, int dtype, int rows, hipStream_t st);
+size_t topps_static_lds();
+hipError_t set_topps_lds_limit(size_t bytes);
 // Batches of greedy rows and rows with 1 <= top_k <= KMAX whose rows fit the
 // top-k kernel's registers (V <= topk_max_vocab(dtype)).
 int topk_max_vocab(int dtype);

@@ -707,8 +707,6 @@ hipError_t launch_sample(const SampleArgs& a, int dtype, size_t lds, hipStream_t
     if (dtype == 1) hipLaunchKernelGGL(full_kernel<uint16_t>, dim3(a.B), blk, lds, st, a);
     else hipLaunchKernelGGL(full_kernel<float>, dim3(a.B), blk, lds, st, a);
     e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    e = launch_topp(a, dtype, st);
   }
   return e;
 }

@@ -39,12 +39,35 @@ struct Elem<uint16_t> {  // bf16 bits
   }
 };
 
+// A 16-byte load of row elements at any element alignment (global memory is
+// in unaligned access mode on this target: one instruction).  NT:
+// non-temporal, for data read once.
+template <bool NT, typename Tin>
+__device__ __forceinline__ uint4 load_row16(const Tin* p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  typedef unsigned v4u __attribute__((ext_vector_type(4)));
+  typedef v4u v4u_a2 __attribute__((aligned(2)));
+  typedef v4u v4u_a4 __attribute__((aligned(4)));
+  v4u t;
+  if constexpr (sizeof(Tin) == 2)
+    t = NT ? __builtin_nontemporal_load((const v4u_a2*)p) : *(const v4u_a2*)p;
+  else
+    t = NT ? __builtin_nontemporal_load((const v4u_a4*)p) : *(const v4u_a4*)p;
+  return make_uint4(t.x, t.y, t.z, t.w);
+#else
+  uint4 t;
+  __builtin_memcpy(&t, p, 16);
+  return t;
+#endif
+}
+
 // Load EPV consecutive logits starting at id v (v a multiple of EPV) from
 // row pointer rowp; ids >= vend read as NaN (never allowed).
 template <typename Tin>
 __device__ __forceinline__ uint4 load_vec(const Tin* rowp, int v, int vend, bool aligned) {
   constexpr int EPV = Elem<Tin>::EPV;
   if (aligned && v + EPV <= vend) return *(const uint4*)(rowp + v);
+  if (v + EPV <= vend) return load_row16<false>(rowp + v);
   uint32_t w[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) w[i] = Elem<Tin>::NAN_BITS;

@@ -1,0 +1,426 @@
+// tgs_topp_split.hip -- rows that sample with top-p over a vocabulary too
+// long for one workgroup's registers (tgs_topp.hip holds those), each row
+// over S workgroups of 512 threads in one launch; in a launch that serves
+// the whole batch, the greedy rows too.
+//
+// What bounds it: one workgroup streams a row at one CU's rate and evaluates
+// every id's exact mass (about 40 VALU operations) on one CU, three passes
+// over the row from L2: 130 - 150 us for a row of 128,256 fp32 or 151,936
+// bf16 ids, whatever the batch, on a chip of 256 CUs.  Here workgroup (b, c)
+// reads ids [c L, (c + 1) L) of row b once, into registers (32 per thread at
+// most), and the row's workgroups meet three times through device memory:
+//
+//   1. Each publishes its chunk's largest composite and polls the row's S of
+//      them: m, the row's maximum.  A poll that runs out (its partners are
+//      not running yet) reads the other chunks itself instead.
+//   2. Each builds the count and mass histogram of its chunk below m in LDS
+//      (tgs_topp.h), stores it to its slab of the workspace, waits for the
+//      stores and counts itself in the row's arrival counter.  The last to
+//      arrive owns the row: it sums the S slabs, places the cut's and the
+//      draw's buckets, and publishes them.
+//   3. The others poll that decision, gather the buckets' ids of their
+//      chunk from registers, publish them and their counts, and leave.  One
+//      whose poll runs out says so and leaves, and the owner reads that
+//      chunk itself (as it does for a chunk with more ids of a bucket than a
+//      list holds).  The owner ranks the lists and finishes the row.
+//
+// No wait depends on a workgroup that has not started: the polls of steps 1
+// and 3 are bounded, and the owner waits only for workgroups that have
+// arrived, whose polls are bounded.  So any grid is safe, whatever else runs
+// on the device; rows are consecutive workgroups, so a row's chunks run
+// together.
+//
+// The exchange uses agent-scope loads and stores throughout (they pass the
+// per-XCD L2s, which are not coherent with each other) and plain waits for
+// the issuing wave's stores; no fence is issued (an agent-scope fence writes
+// back or invalidates a whole L2).  Words carry the call's epoch, so nothing
+// needs clearing between calls except the maxima, whose tag is short.
+//
+// Measured against one workgroup per row streaming it three times (per call):
+// 1 row of 151,936 bf16 ids with penalties 137 -> 30 us, 32 rows of 128,256
+// fp32 ids 141 -> 28 us.  What bounds it now is the chain (stamps of the
+// second, us from the first workgroup's entry): logits in registers 4.7,
+// row's maximum 7.1, histogram 12.1 (the exact exp and two LDS atomics per
+// id), slabs out and counted 13.8, slabs summed 16.0, decision 17.6, lists in
+// 23.2, row written 25.5.  Chunks: at most 16384 ids (32 per thread; more
+// spill), about one workgroup per CU, at least 4096 ids.
+#include "tgs_topp.h"
+
+namespace tgs {
+namespace topp {
+
+constexpr int SBT = TOPPS_NT;
+constexpr uint32_t STAG = 0x3FFFu;    // epoch bits a maximum carries
+constexpr uint32_t SIDM = 0x3FFFFu;   // its id bits (V <= 2^18)
+constexpr uint32_t DONE_LEFT = 1u << 30;  // the chunk's lists were not published
+
+struct SplitShared {
+  Scratch<SBT> ts;
+  BlockScratch bs;
+  u64 rowmax;
+  uint32_t done[TOPPS_MAX_SPLIT];
+  uint32_t arrived, word;
+  int flag;
+};
+
+// Stores of this wave have reached device memory (an agent-scope store is
+// written through, and counts as outstanding until then).
+__device__ __forceinline__ void wait_stores() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+}
+
+template <typename T>
+__device__ __forceinline__ T ld(const T* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void st(T* p, T v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A chunk's largest composite with the epoch's low bits between key and id
+// (never 0; entries of one call order as their composites; key 0: nothing
+// allowed).
+__device__ __forceinline__ u64 max_entry(u64 x, uint32_t ep) {
+  const uint32_t id = x ? (uint32_t)comp_id(x) : 0u;
+  return (x & 0xFFFFFFFF00000000ull) | ((u64)(ep & STAG) << 18) | (u64)(SIDM - id);
+}
+__device__ __forceinline__ bool max_current(u64 e, uint32_t ep) {
+  return e != 0ull && (uint32_t)((e >> 18) & STAG) == (ep & STAG);
+}
+
+// The list buckets in 32 bits (bit 0: they are to be gathered); a run of 32
+// buckets for A or 64 for B is settled by the owner alone.
+__device__ __forceinline__ bool packs(const Plan& pl) { return pl.one && pl.a1 - pl.a0 < 32 && pl.b1 - pl.b0 < 63; }
+__device__ __forceinline__ uint32_t pack_plan(const Plan& pl) {
+  return packs(pl) ? 1u | (uint32_t)pl.a0 << 1 | (uint32_t)(pl.a1 - pl.a0) << 11 | (uint32_t)pl.b0 << 16 |
+                         (uint32_t)(pl.b1 - pl.b0 + 1) << 26
+                   : 0u;
+}
+__device__ __forceinline__ Plan unpack_plan(uint32_t d) {
+  Plan pl;
+  pl.a0 = (int)((d >> 1) & 0x3FFu);
+  pl.a1 = pl.a0 + (int)((d >> 11) & 0x1Fu);
+  pl.b0 = (int)((d >> 16) & 0x3FFu);
+  pl.b1 = pl.b0 + (int)(d >> 26) - 1;
+  return pl;
+}
+
+template <typename Tin>
+__global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
+  TGS_DYN_SMEM(smem);
+  TGS_STATIC_SMEM(SplitShared, sh);
+  using RV = RowView<Tin, true, SBT>;
+  using SV = RowView<Tin, false, SBT>;
+  constexpr int NPRE = RV::NV < TOPP_MASK_PRE ? RV::NV : TOPP_MASK_PRE;
+  const int lb = (int)blockIdx.x / a.S, c = (int)blockIdx.x % a.S;
+  const int b = a.row0 + lb;
+  if (b >= a.B) return;
+  const int w = threadIdx.x >> 6, lane = lane_id();
+  const int v0 = c * a.L, v1 = min(a.V, v0 + a.L);  // a.L a multiple of 64
+  const tgs_row_params p = a.params[b];
+  const float ub = a.u[b];
+  const int hl = a.hist_len ? a.hist_len[b] : a.hist_cap;
+  const Tin* rowp = (const Tin*)a.logits + (long long)b * a.row_stride;
+  // the row's exchange line: counter and epoch, the decision, the chunk
+  // maxima, the done words
+  u64* line = a.tp_lines + (long long)b * TOPPS_LINE;
+  unsigned* cnt = (unsigned*)line;
+  u64* decision = line + 1;
+  u64* maxima = line + 2;
+  u64* done = line + 2 + TOPPS_MAX_SPLIT;
+  const uint32_t epw = ld(cnt + 1);
+  uint4 raw[RV::NV];
+  RV::template fetch<0, NPRE>(rowp, v0, v1, raw);
+  Row r;
+  const bool valid = row_setup_from(a, b, c, p, ub, hl, r);
+  const bool mine = valid && (r.mode == 2 ? !(r.k >= 1 && r.k < a.V) : (r.mode == 0 && a.topp_all));
+  if (!mine) {
+    // other kernels' rows; in a launch that serves the whole batch, invalid
+    // rows (-2) and rows outside the hint (-3)
+    if (a.topp_all && c == 0 && threadIdx.x == 0) {
+      a.out[b] = valid ? -3 : -2;
+      write_row_diag(a, b, 0, 0, 0, 0, -1);
+    }
+    return;
+  }
+  uint32_t mw[RV::NV];
+  RV::mask_words(r, v0, v1, mw);
+  RV::template fetch<NPRE, RV::NV>(rowp, v0, v1, raw);
+  RV::fix_tail(rowp, v0, v1, raw);
+  const uint32_t ep = epw + 1u;  // never 0: the epoch word never holds ~0
+  uint32_t* hbits;
+  int2* hash;
+  int bw;
+  Tail tl = carve(a, smem, hbits, hash, bw);
+  r.v0 = 0;
+  r.v1 = a.V;
+  if (r.use_pen) hash_build<SBT>(a, r, hash, hbits, bw);  // the whole row's: a chunk read again needs them
+  for (int i = threadIdx.x; i < NB + 1; i += SBT) {
+    tl.CI[i] = 0u;
+    tl.MI[i] = 0ull;
+  }
+  Row rc = r;
+  rc.v0 = v0;
+  rc.v1 = v1;
+  RV rv(a, rc, hash, hbits, rowp);
+  rv.load(raw, mw);
+  if (a.dbg.post_logits) {
+    constexpr int EPV = RV::EPV;
+    float* post = a.dbg.post_logits + (long long)b * a.V;
+#pragma unroll
+    for (int q = 0; q < RES_EPT; q++) {
+      const int id = v0 + ((int)threadIdx.x + (q / EPV) * SBT) * EPV + q % EPV;
+      if (id < v1) post[id] = rv.y[q];
+    }
+  }
+
+  // ---- 1. the row's maximum
+  u64 mc = wave_max(thread_best<Tin, SBT>(rv));
+  if (lane == 0) sh.ts.red64[w] = mc;
+  __syncthreads();
+  if (w == 0) {
+    mc = wave_max(lane < SBT / 64 ? sh.ts.red64[lane] : 0ull);
+    if (lane == 0) st(maxima + c, max_entry(mc, ep));
+    const bool act = lane < a.S;
+    u64 e = 0ull;
+    bool ok = false;
+    for (int spins = 0;; spins++) {
+      if (act && !max_current(e, ep)) e = ld(maxima + lane);
+      ok = __ballot(act && !max_current(e, ep)) == 0ull;
+      if (ok || spins >= a.key_spins) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+    // (entries of the call order as their composites)
+    const u64 x = wave_max(act && ok ? e : 0ull);
+    if (lane == 0) {
+      sh.rowmax = (x >> 32) ? comp_key((uint32_t)(x >> 32), (int)(SIDM - (uint32_t)(x & SIDM))) : 0ull;
+      sh.flag = ok;
+    }
+  }
+  __syncthreads();
+  u64 Mc = sh.rowmax;
+  if (!sh.flag) {
+    // the partners are not running: the whole row's maximum from memory
+    SV sv(a, r, hash, hbits, rowp);
+    u64 best = 0ull;
+    sv.each([&](int id, float y) {
+      const u64 x = comp_key(tg_key(y), id);
+      best = x > best ? x : best;
+    });
+    Mc = block_reduce_max<SBT>(best, sh.ts.red64);
+  }
+  tl.m = Mc ? comp_y(Mc) : 0.0f;
+  const bool sampling = Mc != 0ull && r.mode == 2;
+
+  // ---- 2. the chunk's histogram, its slab, and the arrival
+  u64* slab = a.ws + ((long long)lb * a.S + c) * TOPPS_PAIR;
+  if (sampling) {
+    histogram(rv, tl);
+    __syncthreads();
+    unsigned* sc = (unsigned*)(slab + NB);
+    for (int i = threadIdx.x; i < NB; i += SBT) {
+      st(slab + i, tl.MI[i]);
+      st(sc + i, tl.CI[i]);
+    }
+    if (threadIdx.x == 0) st(sc + NB, tl.CI[NB]);
+    wait_stores();
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    sh.arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  const bool owner = sh.arrived == (unsigned)(a.S - 1);
+  if (!owner && !sampling) return;
+
+  if (!owner) {
+    // ---- 3. the decision, and this chunk's ids of its buckets
+    if (w == 0) {
+      u64 d = 0ull;
+      int spins = 0;
+      for (; spins <= a.key_spins; spins++) {
+        d = ld(decision);
+        if ((uint32_t)(d >> 32) == ep) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      if (lane == 0) {
+        sh.flag = (uint32_t)(d >> 32) == ep;
+        sh.word = (uint32_t)d;
+        sh.ts.ng = 0;
+      }
+    }
+    __syncthreads();
+    if (!sh.flag) {
+      if (threadIdx.x == 0) st(done + c, ((u64)ep << 32) | DONE_LEFT);
+      return;
+    }
+    if (!(sh.word & 1u)) return;  // the owner settles the row by itself
+    const Plan pl = unpack_plan(sh.word);
+    u64* list = slab + TOPPS_SLAB;
+    gather(rv, pl, tl.m, sh.ts, [&](int l, unsigned o, u64 x) {
+      if (o < (unsigned)TOPPS_LIST) st(list + l * TOPPS_LIST + o, x);
+    });
+    wait_stores();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const unsigned na = sh.ts.ng & 0xFFFFu, nb = sh.ts.ng >> 16;
+      const bool fit = na <= (unsigned)TOPPS_LIST && nb <= (unsigned)TOPPS_LIST;
+      st(done + c, ((u64)ep << 32) | (fit ? (na << 10) | nb : DONE_LEFT));
+    }
+    return;
+  }
+
+  // ---- the owner: the row's histogram, the cut and the draw
+  if (!sampling) {
+    write_greedy<SBT>(a, r, Mc);
+  } else {
+    const u64* slabs = a.ws + (long long)lb * a.S * TOPPS_PAIR;
+    {
+      // thread t sums buckets t and t + 512, eight slabs' words in flight
+      u64 ms[2] = {0ull, 0ull};
+      unsigned cs[2] = {0u, 0u};
+#pragma unroll 1
+      for (int c0 = 0; c0 < a.S; c0 += 8) {
+        u64 mq[8][2];
+        unsigned cq[8][2];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const u64* s = slabs + (long long)min(c0 + j, a.S - 1) * TOPPS_PAIR;
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            mq[j][h] = ld(s + threadIdx.x + h * SBT);
+            cq[j][h] = ld((const unsigned*)(s + NB) + threadIdx.x + h * SBT);
+          }
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            ms[h] += c0 + j < a.S ? mq[j][h] : 0ull;
+            cs[h] += c0 + j < a.S ? cq[j][h] : 0u;
+          }
+      }
+      static_assert(NB == 2 * SBT, "two buckets per thread");
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        tl.MI[threadIdx.x + h * SBT] = ms[h];
+        tl.CI[threadIdx.x + h * SBT] = cs[h];
+      }
+    }
+    if (w == 0) {
+      unsigned x = lane < a.S ? ld((const unsigned*)(slabs + (long long)lane * TOPPS_PAIR + NB) + NB) : 0u;
+      x = wave_sum(x);
+      if (lane == 0) tl.CI[NB] = x;
+    }
+    __syncthreads();
+    bucket::prefix<SBT>(tl.CI, tl.MI, sh.ts.red32, sh.ts.red64);
+    Plan pl = plan_row<SBT>(r, tl, Mc, tl.CI[NB], sh.ts);
+    if (threadIdx.x == 0)
+      st(decision, ((u64)ep << 32) | pack_plan(pl));
+    SV sv(a, r, hash, hbits, rowp);
+    u64 pick;
+    if (packs(pl)) {
+      auto take = [&](int l, unsigned o, u64 x) { tl.L[l ? pl.ob + o : o] = x; };
+      gather(rv, pl, tl.m, sh.ts, take);
+      if (w == 0) {
+        // every other workgroup of the row has arrived: it publishes its
+        // lists or says that it left, within its own bounded poll
+        const bool act = lane < a.S && lane != c;
+        u64 e = 0ull;
+        for (;;) {
+          if (act && (uint32_t)(e >> 32) != ep) e = ld(done + lane);
+          if (__ballot(act && (uint32_t)(e >> 32) != ep) == 0ull) break;
+          __builtin_amdgcn_s_sleep(1);
+        }
+        if (lane < a.S) sh.done[lane] = act ? (uint32_t)e : 0u;
+      }
+      __syncthreads();
+      // the published lists behind the owner's own, entry t of chunk cc's by
+      // thread cc TPC + t (one round of requests for short lists)
+      const unsigned own = sh.ts.ng;
+      __syncthreads();
+      unsigned pa = own & 0xFFFFu, pb = own >> 16;
+      constexpr unsigned TPC = SBT / TOPPS_MAX_SPLIT;
+      const int mc2 = (int)(threadIdx.x / TPC);
+      unsigned mna = 0u, mnb = 0u, mpa = 0u, mpb = 0u;
+      bool left = false;
+      for (int cc = 0; cc < a.S; cc++) {
+        const uint32_t e = sh.done[cc];
+        if (e & DONE_LEFT) {
+          left = true;
+          continue;
+        }
+        const unsigned na = e >> 10, nb = e & 0x3FFu;
+        if (cc == mc2) {
+          mna = na;
+          mnb = nb;
+          mpa = pa;
+          mpb = pl.ob + pb;
+        }
+        pa += na;
+        pb += nb;
+      }
+      {
+        const u64* list = slabs + (long long)mc2 * TOPPS_PAIR + TOPPS_SLAB;
+        for (unsigned t = threadIdx.x % TPC; t < max(mna, mnb); t += TPC) {
+          const u64 x = t < mna ? ld(list + t) : 0ull;
+          const u64 y = t < mnb ? ld(list + TOPPS_LIST + t) : 0ull;
+          if (t < mna) tl.L[mpa + t] = x;
+          if (t < mnb) tl.L[mpb + t] = y;
+        }
+      }
+      if (left) {  // (uniform)
+        if (threadIdx.x == 0) sh.ts.ng = pa | pb << 16;
+        __syncthreads();
+        for (int cc = 0; cc < a.S; cc++) {
+          if (!(sh.done[cc] & DONE_LEFT)) continue;
+          Row rl = r;
+          rl.v0 = cc * a.L;
+          rl.v1 = min(a.V, rl.v0 + a.L);
+          const SV lv(a, rl, hash, hbits, rowp);
+          gather(lv, pl, tl.m, sh.ts, take);
+        }
+      }
+      __syncthreads();
+      pick = pick_gathered<SBT>(pl, tl, sh.ts, sh.bs);
+    } else {
+      pick = pick_resolved<SBT>(pl, sv, tl, sh.ts, sh.bs);
+    }
+    write_row<SBT>(a, b, pl, pick, sv, sh.ts);
+  }
+  // ready for the next call: counter zero, maxima cleared, epoch advanced
+  // (every workgroup of the row has arrived, so nothing polls the maxima)
+  if (threadIdx.x < (unsigned)a.S) st(maxima + threadIdx.x, (u64)0);
+  if (threadIdx.x == 0) {
+    st(cnt, 0u);
+    st(cnt + 1, ep == 0xFFFFFFFFu ? 0u : ep);
+  }
+}
+
+}  // namespace topp
+
+hipError_t launch_topps(SampleArgs a, int dtype, int rows, hipStream_t st) {
+  const size_t lds = topp_lds_bytes(a.V, a.TS);
+  for (a.row0 = 0; a.row0 < a.B; a.row0 += rows) {
+    const dim3 g((unsigned)((rows < a.B - a.row0 ? rows : a.B - a.row0) * a.S)), blk(TOPPS_NT);
+    if (dtype == 1) hipLaunchKernelGGL((topp::topps_kernel<uint16_t>), g, blk, lds, st, a);
+    else hipLaunchKernelGGL((topp::topps_kernel<float>), g, blk, lds, st, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+size_t topps_static_lds() { return sizeof(topp::SplitShared); }
+
+hipError_t set_topps_lds_limit(size_t bytes) {
+  const hipError_t e1 = hipFuncSetAttribute((const void*)topp::topps_kernel<float>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  const hipError_t e2 = hipFuncSetAttribute((const void*)topp::topps_kernel<uint16_t>,
+                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  return e1 != hipSuccess ? e1 : e2;
+}
+
+}  // namespace tgs
