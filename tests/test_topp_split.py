@@ -1,7 +1,7 @@
-"""Top-p rows over several workgroups (rows longer than one workgroup's
-registers): ragged and padded lengths, both element types, penalties, masks,
-greedy and invalid rows, ties past the ranked capacity, top-p off and near
-zero, infinities and NaN; bit-exact against the oracle.  On the CPU every
+"""Rows over several workgroups (longer than one workgroup's registers): no
+top-k and every kind of top-k, ragged and padded lengths, both element types,
+penalties, masks, greedy and invalid rows, ties past the ranked capacity,
+top-p off and near zero, infinities and NaN; bit-exact against the oracle.  On the CPU every
 workgroup of the launch runs at once (the exchange) or one after another
 (every poll runs out: the fallbacks)."""
 import os
@@ -55,6 +55,43 @@ def _oracle(oracle, x, p, u, h, hl, table):
     return oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=8, want_post=True, nthreads=8)
 
 
+def _topk_rows(oracle, V, seed, bf16=False, mask=False, hist=64):
+    """_rows with a top-k on every sampling row (but the invalid one), and
+    more of them: small and large k, k past the allowed ids of a sparse mask,
+    k that ends in ties, in the mass-0 bucket, above 1024."""
+    x, p, u, h, hl, table = _rows(oracle, V, seed, bf16, mask, hist)
+    p["top_k"] = [50, 1000, 0, 700, 64, 3, 5, 9]
+    g = np.random.default_rng(seed + 1)
+    n = 6
+    rows = [0, 4, 0, 0, 1, 0]
+    x2, p2 = x[rows].copy(), p[rows].copy()
+    p2["top_k"] = [1, 513, 2000, 1024, 7, 512]
+    p2["temperature"] = [1.0, 0.7, 1.3, 0.01, 1.0, 0.6]
+    p2["top_p"] = [0.5, 1.0, 0.8, 1.0, 0.9, 0.999]
+    cat = np.concatenate
+    u2 = (g.integers(0, 1 << 24, n) / (1 << 24)).astype(np.float32)
+    return (cat([x, x2]), cat([p, p2]), cat([u, u2]), None if h is None else cat([h, h[rows]]),
+            None if hl is None else cat([hl, hl[rows]]), table)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("rows,V,bf16,mask,concurrent", [
+    ([0, 1], 32769, False, False, True), ([3, 4], 33001, True, True, True), ([9, 12], 36864, True, False, True),
+    ([8, 10], 32800, False, True, True), ([11, 13], 33000, True, False, True), ([0, 1, 9, 10], 33003, True, False, False),
+    ([4, 11], 33002, False, True, False)])
+def test_topk_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
+    import sim as S
+
+    S.build()
+    x, p, u, h, hl, table = _topk_rows(oracle, V, 9 + V, bf16, mask)
+    x, p, u, h, hl = x[rows], p[rows], u[rows], h[rows], hl[rows]
+    r = S.run_sample(x, p, u, h, hl, mask_table=table, kept_cap=1025, concurrent=concurrent,
+                     env_extra={"TGS_KEY_SPINS": "100000"} if concurrent else None)
+    assert [blk for _, blk in r["launches"]] == [512]  # one launch for every kind of row
+    o = oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=1025, want_post=True, nthreads=8)
+    H.compare(r, o, p, V, what="split top-k")
+
+
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("rows,V,bf16,mask,concurrent", [
     ([0, 1], 32769, False, False, True), ([2, 3], 33001, True, True, True), ([4, 5], 36864, False, True, True),
@@ -81,7 +118,7 @@ def test_split_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
 def test_split_rows(sampler, oracle, V, bf16, mask, hist):
     x, p, u, h, hl, table = _rows(oracle, V, V, bf16, mask, hist)
     o = _oracle(oracle, x, p, u, h, hl, table)
-    for hint in ("auto", None):  # the launch alone, and behind the general kernels
+    for hint in ("auto", None):  # top-p rows and greedy rows alone, and every kind of row
         H.log(f"case split top-p V={V} bf16={bf16} mask={mask} hint={hint}")
         r = H.run_gpu(sampler, x, p, u, h, hl, mask_table=table, kept_cap=8, hint=hint)
         H.compare(r, o, p, V, what="split top-p")
@@ -102,3 +139,30 @@ def test_split_batches(sampler, oracle, B):
         H.log(f"case split top-p batch B={B}")
         r = H.run_gpu(sampler, x, p, u, kept_cap=8, hint="auto")
         H.compare(r, o, p, V, what="split top-p")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,bf16,mask,hist", [
+    (32769, False, False, 64), (32776, True, True, 64), (50001, True, False, 0), (65536, False, True, 1000),
+    (128256, False, False, 64), (128256, True, True, 0), (151935, True, False, 256)])
+def test_topk_rows(sampler, oracle, V, bf16, mask, hist):
+    """Without a hint, with the kept lists and without them (their rows take
+    other lists)."""
+    x, p, u, h, hl, table = _topk_rows(oracle, V, V + 3, bf16, mask, hist)
+    o = oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=1025, want_post=True, nthreads=8)
+    H.log(f"case split top-k V={V} bf16={bf16} mask={mask}")
+    H.compare(H.run_gpu(sampler, x, p, u, h, hl, mask_table=table, kept_cap=1025), o, p, V, what="split top-k")
+    import torch
+
+    import tinygpt_amd as tg
+
+    got = {k: torch.zeros(s, dtype=t, device="cuda:0") for k, s, t in
+           (("counts", (len(p), 2), torch.int32), ("mass", (len(p), 2), torch.int64), ("cut_ids", (len(p),), torch.int32))}
+    ids = sampler.sample(H.to_dev(x), tg.params_to_device(p, "cuda:0"), H.to_dev(u), hist=H.to_dev(h),
+                         hist_len=H.to_dev(hl), vocab=V, debug=got)
+    np.testing.assert_array_equal(ids.cpu().numpy(), o["ids"])
+    ok = o["ids"] != -2
+    np.testing.assert_array_equal(got["counts"].cpu().numpy()[ok], np.stack([o["res"]["n_topk"], o["res"]["n_topp"]], 1)[ok])
+    np.testing.assert_array_equal(got["mass"].cpu().numpy().view(np.uint64)[ok],
+                                  np.stack([o["res"]["mass_k"], o["res"]["mass_p"]], 1)[ok])
+    np.testing.assert_array_equal(got["cut_ids"].cpu().numpy()[ok], o["res"]["cut_id"][ok])

@@ -356,6 +356,9 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     return topp_core(res, err, a, dt, stream);
   }
   a.full_rows = (mk > tgs::KMAX || mk >= V) ? 1 : 0;
+  // rows beyond a workgroup's registers: the split kernel takes every kind
+  if (V > tgs::topp_resident_ids() && tgs::topp_lds_bytes(V, a.TS) + tgs::topps_static_lds() + 256 <= res.lds_limit)
+    return topp_core(res, err, a, dt, stream);
   const int S = choose_split(res.num_cu, res.ws_rows, B, V);
   const int L = S > 1 ? ((V + S - 1) / S + 1023) / 1024 * 1024 : V;
   a.ws_stride = tgs::KMAX;

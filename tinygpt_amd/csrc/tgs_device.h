@@ -448,10 +448,12 @@ __device__ __forceinline__ K block_select_kth(Enum en, unsigned kth, BlockScratc
   return prefix;
 }
 
-// One digit of a mass-weighted radix selection, by one wave: the highest
-// digit d of the 256-bin histogram s.hc / s.hm whose inclusive prefix (from
-// the top, on mass_above) reaches target, into s.sel, with the mass and the
-// count ahead of it (s.mass_above, s.cnt_above) and its own count (s.binc_i).
+// One digit of a radix selection by mass (or by count), by one wave: the
+// highest digit d of the 256-bin histogram s.hc / s.hm whose inclusive prefix
+// (from the top, on what is above) reaches target, into s.sel, with the mass
+// and the count ahead of it (s.mass_above, s.cnt_above) and its own count
+// (s.binc_i).
+template <bool BYCOUNT = false>
 __device__ __forceinline__ void mass_digit_scan(BlockScratch& s, u64 target, u64 mass_above, unsigned cnt_above) {
   const int lane = threadIdx.x;
   unsigned cs[4];
@@ -470,7 +472,7 @@ __device__ __forceinline__ void mass_digit_scan(BlockScratch& s, u64 target, u64
   unsigned ca = 0, bc = 0;
 #pragma unroll
   for (int j = 0; j < 4; j++) {
-    if (found < 0 && cs[j] > 0 && cm + ms[j] >= target) {
+    if (found < 0 && cs[j] > 0 && (BYCOUNT ? (u64)(cc + cs[j]) : cm + ms[j]) >= target) {
       found = 255 - 4 * lane - j;
       ab = cm;
       ca = cc;
@@ -544,10 +546,11 @@ __device__ __forceinline__ u64 block_mass_select(Enum en, u64 target, BlockScrat
 }
 
 // In-place descending bitonic sort of n2 (power of two) keys in LDS.
+template <int BS = NT>
 __device__ __forceinline__ void block_bitonic_desc(u64* buf, int n2) {
   for (int size = 2; size <= n2; size <<= 1) {
     for (int stride = size >> 1; stride > 0; stride >>= 1) {
-      for (int i = threadIdx.x; i < (n2 >> 1); i += NT) {
+      for (int i = threadIdx.x; i < (n2 >> 1); i += BS) {
         const int pos = 2 * i - (i & (stride - 1));
         const int q = pos + stride;
         const bool desc = (pos & size) == 0;

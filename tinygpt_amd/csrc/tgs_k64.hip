@@ -136,44 +136,6 @@ struct HBits {
   __device__ static uint32_t of(const uint32_t* bits, int j) { return (bits[word(j)] >> shift(j)) & GM; }
 };
 
-// max over m = 1 .. NW of the m-th largest of wkey[m - 1][0, NW) (NW one,
-// four or eight), in every lane.  Four waves: lanes 4 (m - 1) + i load
-// wkey[m - 1][i], each group of four lanes sorts itself descending
-// (comparators (0,1) (2,3), (0,2) (1,3), (1,2) as lane exchanges), and lane
-// 5 (m - 1) then holds the m-th largest of group m - 1 (the exchanges are
-// DPP quad permutes).  Eight waves: lanes 8 (m - 1) + i load wkey[m - 1][i],
-// each lane counts the entries of its group that rank above it (larger, or
-// equal at a lower index), and the lane of rank m - 1 in group m - 1 offers
-// its key to a wave maximum.
-template <int NW>
-__device__ __forceinline__ uint32_t bound_key(const uint32_t (*wkey)[NW], int lane) {
-  static_assert(NW == 1 || NW == 4 || NW == 8, "waves per workgroup");
-  if constexpr (NW == 1) {
-    return wkey[0][0];
-  } else if constexpr (NW == 8) {
-    const int g = lane >> 3, i = lane & 7;
-    const uint32_t x = wkey[g][i];
-    int rank = 0;
-#pragma unroll
-    for (int d = 1; d < 8; d++) {
-      const int j = (i + d) & 7;
-      const uint32_t y = __shfl(x, (g << 3) | j, 64);
-      rank += (y > x || (y == x && j < i)) ? 1 : 0;
-    }
-    return wave_max(rank == g ? x : 0u);
-  } else {
-    const int pos = lane & 3;
-    uint32_t x = wkey[(lane >> 2) & 3][pos];
-    uint32_t y = xor_lane32<1>(x);
-    x = (pos & 1) ? min(x, y) : max(x, y);
-    y = xor_lane32<2>(x);
-    x = (pos & 2) ? min(x, y) : max(x, y);
-    y = __builtin_amdgcn_update_dpp(0u, x, 0x1B, 0xF, 0xF, false);  // quad_perm [3,2,1,0]: lane ^ 3
-    x = pos == 1 ? max(x, y) : pos == 2 ? min(x, y) : x;
-    return max(max(readlane_u32(x, 0), readlane_u32(x, 5)), max(readlane_u32(x, 10), readlane_u32(x, 15)));
-  }
-}
-
 // The row's published keys as one wave polls them: lane l holds keys l,
 // l + 64, ... (NJ = ceil(nk / 64) <= 4 of them); keys of this call carry its
 // epoch ep in their high word.  Every slot is loaded (a slot past nk reads
@@ -317,23 +279,6 @@ __device__ __forceinline__ void rank_into(u64* cmp, u64* top, int n, int k) {
     if (act && part == 0 && rk < k) top[rk] = x;
   }
   __syncthreads();
-}
-
-// Tree merge of the waves' sorted top-64 lists (lane i = rank i): after it,
-// wave 0 holds the top 64 of their union, sorted.  Each slot is written once
-// (by its wave, at the level it sends), so one barrier per level suffices.
-// Called by all waves; ends with a barrier.
-template <int NW, typename T>
-__device__ __forceinline__ T merge_waves(T acc, T (*slots)[64]) {
-  const int w = threadIdx.x >> 6, lane = lane_id();
-#pragma unroll
-  for (int step = 1; step < NW; step <<= 1) {
-    if ((w & (2 * step - 1)) == step) slots[w][lane] = acc;
-    __syncthreads();
-    if ((w & (2 * step - 1)) == 0) acc = wave_merge_top64(acc, slots[w + step][lane]);
-  }
-  __syncthreads();
-  return acc;
 }
 
 // The sorted top k of buf[0, n) (n <= CAP, unique composites) in wave 0's

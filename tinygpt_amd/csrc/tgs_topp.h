@@ -254,8 +254,9 @@ struct Tail {
 // 64 are ranked by one wave; more are narrowed first by mass-weighted radix
 // digits from the highest bit in which they differ (one or two passes over
 // the list: counting every entry's rank read n^2 / 2 entries, 5 us at 400).
-// R, Q: 64 entries of scratch.  Ends with a barrier.
-template <int BT>
+// BYCOUNT: the target-th element (target in [1, n]) instead.  R, Q: 64
+// entries of scratch.  Ends with a barrier.
+template <int BT, bool BYCOUNT = false>
 __device__ __forceinline__ u64 select_list(const u64* L, unsigned n, float m, u64 target, u64* before, unsigned* rank,
                                            u64* R, u64* Q, Scratch<BT>& ts, BlockScratch& bs) {
   u64 bm = 0;
@@ -290,7 +291,7 @@ __device__ __forceinline__ u64 select_list(const u64* L, unsigned n, float m, u6
         }
       }
       __syncthreads();
-      if (threadIdx.x < 64) mass_digit_scan(bs, target, bm, br);
+      if (threadIdx.x < 64) mass_digit_scan<BYCOUNT>(bs, target, bm, br);
       __syncthreads();
       bm = bs.mass_above;
       br = bs.cnt_above;
@@ -309,7 +310,7 @@ __device__ __forceinline__ u64 select_list(const u64* L, unsigned n, float m, u6
   }
   if (threadIdx.x < 64) bucket::wave_rank64(L, n, m, R, Q);
   __syncthreads();
-  const int i = bucket::first_rank_once(Q, n, target - bm, &ts.first);
+  const int i = BYCOUNT ? (int)((unsigned)target - br) - 1 : bucket::first_rank_once(Q, n, target - bm, &ts.first);
   *before = bm + (i > 0 ? Q[i - 1] : 0ull);
   *rank = br + (unsigned)i;
   const u64 x = R[i];
@@ -345,10 +346,10 @@ __device__ __forceinline__ u64 resolve_mass(const View& rv, Tail& tl, int bq, u6
 }
 
 // Pass 2: every allowed id of the view into the count and exact-mass
-// histogram over the buckets below m (CI, MI zeroed before).  With a finite
-// maximum, x = y - m is +-0 exactly at y == m, where bucket 0 and weight 1
-// follow from x itself (tg_expf_nonpos(+-0) = 1), so the test for y == m
-// that an infinite maximum needs is left out.
+// histogram over the buckets below m (CI, MI zeroed before).  With
+// a finite maximum, x = y - m is +-0 exactly at y == m, where bucket 0 and
+// weight 1 follow from x itself (tg_expf_nonpos(+-0) = 1), so the test for
+// y == m that an infinite maximum needs is left out.
 template <class View>
 __device__ __forceinline__ void histogram(const View& rv, Tail& tl) {
   const float m = tl.m;
@@ -376,18 +377,19 @@ __device__ __forceinline__ void histogram(const View& rv, Tail& tl) {
 
 // Where a row's cut and draw lie, from the inclusive prefixes.
 struct Plan {
-  u64 S, P, Sp;         // kept mass, the top-p target, S' (final unless cut_search)
-  u64 cutc;             // the cut's composite (final unless cut_search)
-  unsigned ntopp, nv;   // size of the top-p set (final unless cut_search), allowed ids
-  uint32_t uq;          // floor(u 2^24)
-  bool cut_search;      // the cut is an element of bucket bp still to be found
-  bool cut_last;        // top-p off: the cut is the smallest allowed composite
-  bool one;             // lists A and B fit: one gather settles the row
-  int bp;               // the cut's bucket
-  int a0, a1;           // list A's buckets
-  int b0, b1;           // list B's buckets (b0 > b1: none)
-  unsigned na, nb;      // their ids
-  unsigned ob;          // list B's offset in the lists
+  u64 S = 0, P = 0, Sp = 0;  // kept mass, the top-p target, S' (final unless cut_search)
+  u64 cutc = 0;  // the cut's composite (final unless cut_search)
+  unsigned ntopp = 0, nv = 0;  // size of the top-p set (final unless cut_search), of the top-k set (all allowed ids without one)
+  uint32_t uq = 0;  // floor(u 2^24)
+  bool cut_search = false;  // the cut is an element of bucket bp still to be found
+  bool cut_last = false;  // top-p off: the cut is the top-k set's last element
+  bool k_search = false;  // the top-k set ends inside list A: S, and what follows from it, is settled there
+  bool one = false;  // lists A and B fit: one gather settles the row
+  int bp = 0;  // the cut's bucket (k_search: the top-k set's last)
+  int a0 = 0, a1 = 0;  // list A's buckets
+  int b0 = 1, b1 = 0;  // list B's buckets (b0 > b1: none)
+  unsigned na = 0, nb = 0;  // their ids
+  unsigned ob = 0;  // list B's offset in the lists
   // which list bucket q belongs to: 0 A, 1 B, -1 neither
   __device__ __forceinline__ int list(int q) const {
     return q >= a0 && q <= a1 ? 0 : q >= b0 && q <= b1 ? 1 : -1;
@@ -402,33 +404,35 @@ struct Plan {
 // they meet it, else as list B (a run of buckets ranks like one).  Zeroes the
 // list counters; ends with a barrier.
 template <int BT>
-__device__ __forceinline__ Plan plan_row(const Row& r, const Tail& tl, u64 Mc, unsigned nv, Scratch<BT>& ts) {
-  Plan pl;
-  pl.S = tl.MI[NB - 1];
+__device__ __forceinline__ void plan_row(Plan& pl, const Row& r, const Tail& tl, u64 Mc, unsigned nv, Scratch<BT>& ts) {
+  const u64 S = tl.MI[NB - 1];
+  u64 P = 0, Sp = S, low = S;  // low: the least S' can be
   pl.cutc = 0;
-  pl.Sp = pl.S;
-  pl.P = 0;
   pl.ntopp = nv;
   pl.nv = nv;
   pl.cut_last = false;
   pl.cut_search = false;
+  pl.k_search = false;
   if (r.top_p < 1.0f) {
-    const uint32_t pq = (uint32_t)(r.top_p * 16777216.0f);
-    pl.P = mul_shr24(pl.S, pq);
-    if (pl.P == 0) {
+    P = mul_shr24(S, (uint32_t)(r.top_p * 16777216.0f));
+    if (P == 0) {
       pl.cutc = Mc;
-      pl.Sp = tg_q40(1.0f);
+      low = Sp = tg_q40(1.0f);
       pl.ntopp = 1;
     } else {
       pl.cut_search = true;
+      low = P;
     }
   } else {
     pl.cut_last = true;
   }
+  pl.S = S;
+  pl.P = P;
+  pl.Sp = Sp;
   pl.uq = (uint32_t)(r.u * 16777216.0f);
-  const u64 tlo = mul_shr24(pl.cut_search ? pl.P : pl.Sp, pl.uq);
+  const u64 tlo = mul_shr24(low, pl.uq);
   if (threadIdx.x == 0) ts.ng = 0;
-  bucket::find_mass2<BT>(tl.MI, pl.cut_search ? pl.P : tlo + 1, tlo + 1, &ts.sel[0], &ts.sel[1]);
+  bucket::find_mass2<BT>(tl.MI, pl.cut_search ? low : tlo + 1, tlo + 1, &ts.sel[0], &ts.sel[1]);
   pl.bp = ts.sel[0];
   const int btl = ts.sel[1];
   int bth = btl;
@@ -445,7 +449,61 @@ __device__ __forceinline__ Plan plan_row(const Row& r, const Tail& tl, u64 Mc, u
   pl.nb = join ? 0u : tl.CI[bth] - bucket::count_before(tl.CI, btl);
   pl.ob = pl.na;
   pl.one = pl.na + pl.nb <= (unsigned)CAPL;
-  return pl;
+}
+
+// The same for a row whose top-k set (its kk first allowed ids, kk below the
+// allowed count) ends in bucket bk < NB.  S lies in [slo, MI[bk]] (all of the
+// buckets before bk, and the maximum's own mass), and P, S' and the draw's
+// target follow with it, so list A runs from the lowest bucket the cut can
+// lie in to bk, joined by the draw's run when they meet.  Ends with a
+// barrier.
+template <int BT>
+__device__ __forceinline__ void plan_topk(Plan& pl, const Row& r, const Tail& tl, u64 Mc, unsigned kk,
+                                          Scratch<BT>& ts) {
+  pl.nv = kk;
+  pl.ntopp = kk;
+  pl.cutc = 0;
+  pl.k_search = true;
+  pl.cut_search = pl.cut_last = false;
+  if (threadIdx.x == 0) ts.ng = 0;
+  const int bk = bucket::find_count<BT>(tl.CI, kk, &ts.sel[0]);
+  pl.bp = bk;
+  const u64 one = tg_q40(1.0f), sb = bucket::mass_before(tl.MI, bk);
+  const u64 slo = sb > one ? sb : one, shi = tl.MI[bk];
+  pl.S = shi;
+  pl.uq = (uint32_t)(r.u * 16777216.0f);
+  const uint32_t pq = r.top_p < 1.0f ? (uint32_t)(r.top_p * 16777216.0f) : 0u;
+  pl.P = 0;
+  pl.Sp = one;
+  u64 plo = slo, phi = shi;  // the range of S'
+  int lo = bk;
+  if (r.top_p < 1.0f && pq == 0u) {
+    pl.cutc = Mc;
+    pl.ntopp = 1;
+    plo = phi = one;
+  } else if (r.top_p < 1.0f) {
+    pl.cut_search = true;
+    plo = mul_shr24(slo, pq);  // >= 1: slo >= 2^40
+    phi = mul_shr24(shi, pq);
+    bucket::find_mass2<BT>(tl.MI, plo, phi, &ts.sel[1], &ts.sel[2]);
+    lo = ts.sel[1] < bk ? ts.sel[1] : bk;
+    phi = tl.MI[ts.sel[2] < bk ? ts.sel[2] : bk];
+    __syncthreads();  // before the slots are written again
+  } else {
+    pl.cut_last = true;
+  }
+  bucket::find_mass2<BT>(tl.MI, mul_shr24(plo, pl.uq) + 1, mul_shr24(phi, pl.uq) + 1, &ts.sel[1], &ts.sel[2]);
+  const int dl = ts.sel[1], dh = ts.sel[2] < bk ? ts.sel[2] : bk;
+  const bool join = dh >= lo;
+  if (join && dl < lo) lo = dl;
+  pl.a0 = lo;
+  pl.a1 = bk;
+  pl.b0 = join ? 1 : dl;
+  pl.b1 = join ? 0 : dh;
+  pl.na = tl.CI[bk] - bucket::count_before(tl.CI, lo);
+  pl.nb = pl.b0 <= pl.b1 ? tl.CI[pl.b1] - bucket::count_before(tl.CI, pl.b0) : 0u;
+  pl.ob = pl.na;
+  pl.one = pl.na + pl.nb <= (unsigned)CAPL;
 }
 
 // The allowed ids of the lists' buckets, in no particular order, into their
@@ -483,6 +541,26 @@ __device__ __forceinline__ void gather(const RowView<Tin, true, BT>& rv, const P
     else sink(1, ob++, x);
   }
 }
+// The allowed ids with y >= yb, in no particular order (sink(place,
+// composite)); ts.ng counts them (zero before).  The same marks and places.
+template <typename Tin, int BT, class F>
+__device__ __forceinline__ void gather_floor(const RowView<Tin, true, BT>& rv, float yb, Scratch<BT>& ts, F sink) {
+  constexpr int EPV = Elem<Tin>::EPV;
+  uint32_t ma = 0u;
+#pragma unroll
+  for (int q = 0; q < RES_EPT; q++) ma |= (rv.y[q] >= yb && rv.y[q] > -__builtin_inff()) ? 1u << q : 0u;
+  const unsigned n = (unsigned)__popc(ma);
+  const unsigned incl = wave_incl_scan(n);
+  const unsigned tot = readlane_u32(incl, 63);
+  if (tot == 0u) return;
+  unsigned at = 0u;
+  if (lane_id() == 0) at = atomicAdd(&ts.ng, tot);
+  at = readlane_u32(at, 0) + incl - n;
+#pragma unroll
+  for (int q = 0; q < RES_EPT; q++)
+    if ((ma >> q) & 1u)
+      sink(at++, comp_key(tg_key(rv.y[q]), rv.r.v0 + ((int)threadIdx.x + (q / EPV) * BT) * EPV + q % EPV));
+}
 // From any other view: one at a time.
 template <class View, int BT, class F>
 __device__ __forceinline__ void gather(const View& rv, const Plan& pl, float m, Scratch<BT>& ts, F sink) {
@@ -498,8 +576,9 @@ __device__ __forceinline__ void gather(const View& rv, const Plan& pl, float m, 
 // between the gather and the call); settles the cut.  Lists of at most 64
 // ids are ranked side by side by two waves.
 template <int BT>
-__device__ __forceinline__ u64 pick_gathered(Plan& pl, Tail& tl, Scratch<BT>& ts, BlockScratch& bs) {
+__device__ __forceinline__ u64 pick_gathered(Plan& pl, float top_p, Tail& tl, Scratch<BT>& ts, BlockScratch& bs) {
   const float m = tl.m;
+  u64 P = pl.P, Sp = pl.Sp;
   const int w = (int)threadIdx.x >> 6;
   const bool ra = pl.na <= 64u, rb = pl.nb <= 64u;  // (uniform)
   if (ra && w == 0) bucket::wave_rank64(tl.L, pl.na, m, tl.R, tl.Q);
@@ -508,8 +587,26 @@ __device__ __forceinline__ u64 pick_gathered(Plan& pl, Tail& tl, Scratch<BT>& ts
   u64 before;
   unsigned rank;
   const u64 before_a = bucket::mass_before(tl.MI, pl.a0);
+  if (pl.k_search) {
+    // the top-k set's last element: S, then P or S'
+    const unsigned ik = pl.nv - bucket::count_before(tl.CI, pl.a0);  // its place in list A
+    u64 last;
+    if (ra) {
+      last = tl.R[ik - 1];
+      pl.S = before_a + tl.Q[ik - 1];
+    } else {
+      last = select_list<BT, true>(tl.L, pl.na, m, ik, &before, &rank, tl.R, tl.Q, ts, bs);
+      pl.S = before_a + before + bucket::mass_c(last, m);
+    }
+    if (pl.cut_last) {
+      pl.cutc = last;
+      Sp = pl.S;
+    } else if (pl.cut_search) {
+      P = mul_shr24(pl.S, (uint32_t)(top_p * 16777216.0f));
+    }
+  }
   if (pl.cut_search) {
-    const u64 target = pl.P - before_a;
+    const u64 target = P - before_a;
     if (ra) {
       const int i = bucket::first_rank_once(tl.Q, pl.na, target, &ts.first2);
       pl.cutc = tl.R[i];
@@ -518,10 +615,11 @@ __device__ __forceinline__ u64 pick_gathered(Plan& pl, Tail& tl, Scratch<BT>& ts
     } else {
       pl.cutc = select_list<BT>(tl.L, pl.na, m, target, &before, &rank, tl.R, tl.Q, ts, bs);
     }
-    pl.Sp = before_a + before + bucket::mass_c(pl.cutc, m);
+    Sp = before_a + before + bucket::mass_c(pl.cutc, m);
     pl.ntopp = bucket::count_before(tl.CI, pl.a0) + rank + 1u;
   }
-  const u64 t = mul_shr24(pl.Sp, pl.uq);
+  pl.Sp = Sp;
+  const u64 t = mul_shr24(Sp, pl.uq);
   if (pl.nb > 0u) {
     const u64 target = t + 1 - bucket::mass_before(tl.MI, pl.b0);
     if (rb) return tl.R2[bucket::first_rank_once(tl.Q2, pl.nb, target, &ts.first)];
@@ -548,11 +646,12 @@ __device__ __forceinline__ u64 pick_resolved(Plan& pl, const View& rv, Tail& tl,
   return resolve_mass<BT>(rv, tl, bt, t + 1 - bucket::mass_before(tl.MI, bt), &before, &rank, ts, bs);
 }
 
-// The id and the diagnostics of a settled sampling row.
+// The id and the diagnostics of a settled sampling row without a top-k, or
+// with one above KMAX (no kept list).
 template <int BT, class View>
 __device__ __forceinline__ void write_row(const SampleArgs& a, int b, Plan& pl, u64 pick, const View& rv,
                                           Scratch<BT>& ts) {
-  if (pl.cut_last && a.dbg.cut_ids) {
+  if (pl.cut_last && !pl.k_search && a.dbg.cut_ids) {
     u64 x = 0;
     rv.each([&](int id, float y) {
       const u64 v = ~comp_key(tg_key(y), id);
@@ -568,6 +667,67 @@ __device__ __forceinline__ void write_row(const SampleArgs& a, int b, Plan& pl, 
     for (int i = threadIdx.x; i < a.dbg.kept_cap; i += BT) a.dbg.kept_ids[(long long)b * a.dbg.kept_cap + i] = -1;
   if (a.dbg.kept_probs)
     for (int i = threadIdx.x; i < a.dbg.kept_cap; i += BT) a.dbg.kept_probs[(long long)b * a.dbg.kept_cap + i] = 0.0f;
+}
+
+// The kept list of a row with 1 <= top_k <= KMAX: sorted[0, n) its top-k set
+// in order, the first ntopp of them with their probabilities.
+template <int BT>
+__device__ __forceinline__ void write_kept(const SampleArgs& a, int b, const u64* sorted, int n, int ntopp, u64 Sp,
+                                           float m) {
+  if (a.dbg.kept_ids) {
+    int32_t* kid = a.dbg.kept_ids + (long long)b * a.dbg.kept_cap;
+    for (int i = threadIdx.x; i < a.dbg.kept_cap; i += BT) kid[i] = i < n ? comp_id(sorted[i]) : -1;
+  }
+  if (a.dbg.kept_probs) {
+    float* kp = a.dbg.kept_probs + (long long)b * a.dbg.kept_cap;
+    const float fs = tg_u64_to_f32(Sp);
+    for (int i = threadIdx.x; i < a.dbg.kept_cap; i += BT)
+      kp[i] = i < ntopp ? kept_prob(comp_y(sorted[i]), m, fs) : 0.0f;
+  }
+}
+
+// The row settled without the lists, by radix selections over the view read
+// again for every digit: a top-k of kk elements out of more allowed ids, any
+// ties.
+template <int BT, class View>
+__device__ __forceinline__ u64 pick_streamed(Plan& pl, unsigned kk, const Row& r, const View& sv, u64 Mc, Tail& tl,
+                                             Scratch<BT>& ts, BlockScratch& bs) {
+  const float m = tl.m;
+  pl.uq = (uint32_t)(r.u * 16777216.0f);
+  const u64 T = block_select_kth<u64, 64, BT>(
+      [&](auto f) { sv.each([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, kk, bs);
+  auto each_kept = [&](auto f) {
+    sv.each([&](int id, float y) {
+      const u64 x = comp_key(tg_key(y), id);
+      if (x >= T) f(x, bucket::mass(y, m));
+    });
+  };
+  u64 S = 0, minc = ~0ull;
+  each_kept([&](u64 x, u64 q) {
+    S += q;
+    minc = x < minc ? x : minc;
+  });
+  S = block_sum<u64, BT>(S, ts.red64);
+  minc = ~block_max<u64, BT>(~minc, ts.red64b);
+  u64 before;
+  unsigned rank;
+  pl.nv = pl.ntopp = kk;
+  pl.S = pl.Sp = S;
+  pl.cutc = minc;
+  pl.k_search = pl.cut_last = true;  // the cut is settled
+  if (r.top_p < 1.0f) {
+    pl.P = mul_shr24(S, (uint32_t)(r.top_p * 16777216.0f));
+    if (pl.P == 0) {
+      pl.cutc = Mc;
+      pl.Sp = tg_q40(1.0f);
+      pl.ntopp = 1;
+    } else {
+      pl.cutc = block_mass_select<BT>(each_kept, pl.P, bs, &before, &rank);
+      pl.Sp = before + bucket::mass_c(pl.cutc, m);
+      pl.ntopp = rank + 1;
+    }
+  }
+  return block_mass_select<BT>(each_kept, mul_shr24(pl.Sp, pl.uq) + 1, bs, &before, &rank);
 }
 
 // A greedy row (the largest composite Mc), or a row with nothing allowed

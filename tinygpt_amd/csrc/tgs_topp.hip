@@ -46,12 +46,13 @@ __device__ __forceinline__ void topp_rest(const SampleArgs& a, const Row& r, con
   histogram(rv, tl);
   __syncthreads();
   bucket::prefix<BT>(tl.CI, tl.MI, ts.red32, ts.red64);
-  Plan pl = plan_row<BT>(r, tl, Mc, nv, ts);
+  Plan pl;
+  plan_row<BT>(pl, r, tl, Mc, nv, ts);
   u64 pick;
   if (pl.one) {
     gather(rv, pl, tl.m, ts, [&](int l, unsigned o, u64 x) { tl.L[l ? pl.ob + o : o] = x; });
     __syncthreads();
-    pick = pick_gathered<BT>(pl, tl, ts, bs);
+    pick = pick_gathered<BT>(pl, r.top_p, tl, ts, bs);
   } else {
     pick = pick_resolved<BT>(pl, rv, tl, ts, bs);
   }

@@ -59,7 +59,11 @@ struct SplitShared {
   BlockScratch bs;
   u64 rowmax;
   uint32_t done[TOPPS_MAX_SPLIT];
-  uint32_t arrived, word;
+  uint32_t wkey[2][SBT / 64][SBT / 64];  // per bound: [m - 1][wave]: the wave's ceil(k / m)-th largest thread maximum
+  u64 slots[SBT / 64][64];               // wave lists (the ranked top-k of at most 64)
+  uint32_t floor;
+  u64 word;
+  uint32_t arrived;
   int flag;
 };
 
@@ -91,22 +95,148 @@ __device__ __forceinline__ bool max_current(u64 e, uint32_t ep) {
   return e != 0ull && (uint32_t)((e >> 18) & STAG) == (ep & STAG);
 }
 
-// The list buckets in 32 bits (bit 0: they are to be gathered); a run of 32
-// buckets for A or 64 for B is settled by the owner alone.
-__device__ __forceinline__ bool packs(const Plan& pl) { return pl.one && pl.a1 - pl.a0 < 32 && pl.b1 - pl.b0 < 63; }
-__device__ __forceinline__ uint32_t pack_plan(const Plan& pl) {
-  return packs(pl) ? 1u | (uint32_t)pl.a0 << 1 | (uint32_t)(pl.a1 - pl.a0) << 11 | (uint32_t)pl.b0 << 16 |
-                         (uint32_t)(pl.b1 - pl.b0 + 1) << 26
-                   : 0u;
+// The composite of the largest entry (0: nothing allowed).
+__device__ __forceinline__ u64 max_comp(u64 e) {
+  return (e >> 32) ? comp_key((uint32_t)(e >> 32), (int)(SIDM - (uint32_t)(e & SIDM))) : 0ull;
 }
-__device__ __forceinline__ Plan unpack_plan(uint32_t d) {
+
+// Ready for the next call: counter zero, maxima cleared, epoch advanced
+// (every workgroup of the row has arrived, so nothing polls the maxima).
+__device__ __forceinline__ void reset_line(const SampleArgs& a, unsigned* cnt, u64* maxima, uint32_t ep) {
+  if (threadIdx.x < (unsigned)a.S) st(maxima + threadIdx.x, (u64)0);
+  if (threadIdx.x == 0) {
+    st(cnt, 0u);
+    st(cnt + 1, ep == 0xFFFFFFFFu ? 0u : ep);
+  }
+}
+
+// A wave polls the row's S words (one per chunk) until each is current;
+// false after max_spins polls.  *e: lane c's word.
+__device__ __forceinline__ bool poll_words(const u64* words, int S, uint32_t ep, int max_spins, u64* e) {
+  const bool act = lane_id() < S;
+  u64 x = 0ull;
+  bool ok = false;
+  for (int spins = 0;; spins++) {
+    if (act && !max_current(x, ep)) x = ld(words + lane_id());
+    ok = __ballot(act && !max_current(x, ep)) == 0ull;
+    if (ok || spins >= max_spins) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+  *e = act ? x : 0ull;
+  return ok;
+}
+
+// Two floor keys (their top 23 bits: a floor may be lower) in one word with
+// the epoch's tag where max_current looks for it.
+__device__ __forceinline__ u64 floor_entry(uint32_t k1, uint32_t k2, uint32_t ep) {
+  return (u64)(k1 >> 9) << 41 | (u64)((k2 >> 9) >> 14) << 32 | (u64)(ep & STAG) << 18 | (u64)(((k2 >> 9) & 0x3FFFu) << 4) | 1ull;
+}
+__device__ __forceinline__ uint32_t floor_key1(u64 e) { return (uint32_t)(e >> 41) << 9; }
+__device__ __forceinline__ uint32_t floor_key2(u64 e) {
+  return (((uint32_t)(e >> 32) & 0x1FFu) << 14 | ((uint32_t)e >> 4 & 0x3FFFu)) << 9;
+}
+
+// The sorted top 64 of L[0, n) in wave 0's lanes (slots: the waves' lists).
+// Ends with a barrier.
+__device__ __forceinline__ u64 top64(const u64* L, unsigned n, u64 (*slots)[64]) {
+  u64 acc = 0ull;
+  bool first = true;
+  for (unsigned s0 = threadIdx.x & ~63u; s0 < n; s0 += SBT) {
+    u64 x = s0 + lane_id() < n ? L[s0 + lane_id()] : 0ull;
+    x = wave_sort_desc(x);
+    acc = first ? x : wave_merge_top64(acc, x);
+    first = false;
+  }
+  return merge_waves<SBT / 64>(acc, slots);
+}
+
+// A row with 1 <= top_k <= KMAX from L[0, n), which holds its top-k set (n <=
+// CAPL; every allowed id when fewer than k are): finished by one wave up to
+// 64 kept ids; otherwise the set is cut out of the list by its k-th element,
+// and the cut and the draw selected by mass.
+__device__ __forceinline__ void finish_topk(const SampleArgs& a, const Row& r, u64* L, unsigned n, Tail& tl,
+                                            SplitShared& sh) {
+  const unsigned k = (unsigned)r.k, kk = k < n ? k : n;
+  if (kk <= 64u) {
+    const u64 x = top64(L, n, sh.slots);
+    if (threadIdx.x < 64) wave_finalize(a, r, (unsigned)lane_id() < kk ? x : 0ull, (int)kk);
+    return;
+  }
+  constexpr int PER = (CAPL + SBT - 1) / SBT;
+  u64 mx = 0ull;
+  for (unsigned i = threadIdx.x; i < n; i += SBT) mx = L[i] > mx ? L[i] : mx;
+  const u64 Mc = block_reduce_max<SBT>(mx, sh.ts.red64);
+  const float m = comp_y(Mc);
+  u64 before = 0;
+  unsigned rank = 0;
+  unsigned ntopp = kk;
+  u64 T = 0ull;
+  if (kk < n) T = select_list<SBT, true>(L, n, m, kk, &before, &rank, tl.R, tl.Q, sh.ts, sh.bs);
+  u64 keep[PER];
+  u64 S = 0, mn = ~0ull;
+#pragma unroll
+  for (int j = 0; j < PER; j++) {
+    const unsigned i = threadIdx.x + j * SBT;
+    keep[j] = i < n ? L[i] : 0ull;
+    if (keep[j] < T) keep[j] = 0ull;
+    if (keep[j]) {
+      S += bucket::mass_c(keep[j], m);
+      mn = keep[j] < mn ? keep[j] : mn;
+    }
+  }
+  if (threadIdx.x == 0) sh.ts.ng = 0;
+  const u64 St = block_sum<u64, SBT>(S, sh.ts.red64);  // (its barriers also end the reads of L)
+  u64 cutc = ~block_max<u64, SBT>(~mn, sh.ts.red64b);
+#pragma unroll
+  for (int j = 0; j < PER; j++)
+    if (keep[j]) L[atomicAdd(&sh.ts.ng, 1u)] = keep[j];
+  __syncthreads();
+  u64 Sp = St;
+  if (r.top_p < 1.0f) {
+    const u64 P = mul_shr24(St, (uint32_t)(r.top_p * 16777216.0f));
+    if (P == 0) {
+      cutc = Mc;
+      Sp = tg_q40(1.0f);
+      ntopp = 1;
+    } else {
+      cutc = select_list<SBT>(L, kk, m, P, &before, &rank, tl.R, tl.Q, sh.ts, sh.bs);
+      Sp = before + bucket::mass_c(cutc, m);
+      ntopp = rank + 1;
+    }
+  }
+  const u64 t = mul_shr24(Sp, (uint32_t)(r.u * 16777216.0f));
+  const u64 pick = select_list<SBT>(L, kk, m, t + 1, &before, &rank, tl.R, tl.Q, sh.ts, sh.bs);
+  if (threadIdx.x == 0) {
+    a.out[r.b] = comp_id(pick);
+    write_row_diag(a, r.b, (int)kk, (int)ntopp, St, Sp, comp_id(cutc));
+  }
+  if (a.dbg.kept_ids || a.dbg.kept_probs) {
+    int n2 = 1;
+    while (n2 < (int)kk) n2 <<= 1;
+    for (int i = (int)kk + (int)threadIdx.x; i < n2; i += SBT) L[i] = 0ull;
+    __syncthreads();
+    block_bitonic_desc<SBT>(L, n2);
+    write_kept<SBT>(a, r.b, L, (int)kk, (int)ntopp, Sp, m);
+  }
+}
+
+// The decision word: the epoch's low 24 bits over the list buckets in 40
+// (bit 0: they are to be gathered; a run of 512 buckets or more for list B is
+// settled by the owner alone).  Every call of a row writes it, so a stale one
+// is the previous call's.
+__device__ __forceinline__ bool packs(const Plan& pl) { return pl.one && pl.b1 - pl.b0 < 511; }
+__device__ __forceinline__ u64 pack_plan(const Plan& pl) {
+  return 1ull | (u64)pl.a0 << 1 | (u64)pl.a1 << 11 | (u64)pl.b0 << 21 | (u64)(pl.b1 - pl.b0 + 1) << 31;
+}
+__device__ __forceinline__ Plan unpack_plan(u64 d) {
   Plan pl;
   pl.a0 = (int)((d >> 1) & 0x3FFu);
-  pl.a1 = pl.a0 + (int)((d >> 11) & 0x1Fu);
-  pl.b0 = (int)((d >> 16) & 0x3FFu);
-  pl.b1 = pl.b0 + (int)(d >> 26) - 1;
+  pl.a1 = (int)((d >> 11) & 0x3FFu);
+  pl.b0 = (int)((d >> 21) & 0x3FFu);
+  pl.b1 = pl.b0 + (int)((d >> 31) & 0x1FFu) - 1;
   return pl;
 }
+__device__ __forceinline__ bool decided(u64 d, uint32_t ep) { return (uint32_t)(d >> 40) == (ep & 0xFFFFFFu); }
 
 template <typename Tin>
 __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
@@ -136,11 +266,10 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   RV::template fetch<0, NPRE>(rowp, v0, v1, raw);
   Row r;
   const bool valid = row_setup_from(a, b, c, p, ub, hl, r);
-  const bool mine = valid && (r.mode == 2 ? !(r.k >= 1 && r.k < a.V) : (r.mode == 0 && a.topp_all));
-  if (!mine) {
-    // other kernels' rows; in a launch that serves the whole batch, invalid
-    // rows (-2) and rows outside the hint (-3)
-    if (a.topp_all && c == 0 && threadIdx.x == 0) {
+  const bool has_k = r.k >= 1 && r.k < a.V;
+  const bool mine = valid && (a.topp_all ? r.mode == 0 || (r.mode == 2 && !has_k) : !outside_hint(a, r));
+  if (!mine) {  // invalid rows (-2) and rows outside the hint (-3)
+    if (c == 0 && threadIdx.x == 0) {
       a.out[b] = valid ? -3 : -2;
       write_row_diag(a, b, 0, 0, 0, 0, -1);
     }
@@ -177,26 +306,151 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
   }
 
+  u64 mc = thread_best<Tin, SBT>(rv);
+  u64* slab = a.ws + ((long long)lb * a.S + c) * TOPPS_PAIR;
+  const u64* slabs = a.ws + (long long)lb * a.S * TOPPS_PAIR;
+  if (threadIdx.x == 0) sh.ts.ng = 0;
+
+  if (r.mode == 1) {
+    // ---- a top-k of at most KMAX: the chunk's ids that reach a floor under
+    // the row's k-th largest y, and no more meetings.  Floors from the thread
+    // maxima (bound_key): the chunk's own k-th largest (k <= SBT), or, when S
+    // lists of that many would be too long (meet), the lowest over the chunks
+    // of each one's ceil(k / S)-th largest, or the highest of their k-th.
+    const bool meet = 2 * a.S * r.k > CAPL;
+    const int k2 = (r.k + a.S - 1) / a.S;
+    const uint32_t srt = wave_sort_desc((uint32_t)(mc >> 32));
+#pragma unroll
+    for (int q = 1; q <= SBT / 64; q++) {
+      const int at = (r.k + q - 1) / q - 1, at2 = (k2 + q - 1) / q - 1;
+      const uint32_t x = readlane_u32(srt, at & 63), x2 = readlane_u32(srt, at2 & 63);
+      if (lane == 0) {
+        sh.wkey[0][q - 1][w] = at < 64 ? x : 0u;
+        sh.wkey[1][q - 1][w] = at2 < 64 ? x2 : 0u;
+      }
+    }
+    __syncthreads();
+    uint32_t kb = bound_key<SBT / 64>(sh.wkey[0], lane);
+    if (meet) {
+      if (w == 0) {
+        const uint32_t kb2 = bound_key<SBT / 64>(sh.wkey[1], lane);
+        if (lane == 0) st(maxima + c, floor_entry(kb2, kb, ep));
+        u64 e;
+        const bool ok = poll_words(maxima, a.S, ep, a.key_spins, &e);
+        const uint32_t lo = ~wave_max(lane < a.S ? ~floor_key1(e) : 0u), hi = wave_max(lane < a.S ? floor_key2(e) : 0u);
+        if (lane == 0) sh.floor = ok ? (lo > hi ? lo : hi) : 0u;
+      }
+      __syncthreads();
+      kb = sh.floor > kb ? sh.floor : kb;
+    }
+    const float yb = kb ? tg_unkey(kb) : -__builtin_inff();
+    gather_floor(rv, yb, sh.ts, [&](unsigned o, u64 x) {
+      if (o < (unsigned)TOPPS_PAIR) st(slab + o, x);
+    });
+    wait_stores();
+    __syncthreads();
+    unsigned n = sh.ts.ng;
+    if (n > (unsigned)TOPPS_PAIR) {
+      // more ids than the list holds (ties at the floor, no floor): the
+      // chunk's exact top k, read again
+      const SV cv(a, rc, hash, hbits, rowp);
+      const u64 T = block_select_kth<u64, 64, SBT>(
+          [&](auto f) { cv.each([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, (unsigned)r.k, sh.bs);
+      if (threadIdx.x == 0) sh.ts.ng = 0;
+      __syncthreads();
+      cv.each([&](int id, float y) {
+        const u64 x = comp_key(tg_key(y), id);
+        if (x >= T) st(slab + atomicAdd(&sh.ts.ng, 1u), x);
+      });
+      wait_stores();
+      __syncthreads();
+      n = sh.ts.ng;
+    }
+    if (threadIdx.x == 0) {
+      st(done + c, ((u64)ep << 32) | n);
+      wait_stores();
+      sh.arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (sh.arrived != (unsigned)(a.S - 1)) return;
+    // the owner: every list has been published
+    if (w == 0) {
+      const bool act = lane < a.S;
+      const uint32_t incl = wave_incl_scan(act ? (uint32_t)ld(done + lane) : 0u);
+      if (act) sh.done[lane] = incl;
+    }
+    __syncthreads();
+    n = sh.done[a.S - 1];
+    // f(entry i) for this thread's share of the lists laid end to end
+    auto each_entry = [&](auto f) {
+      for (unsigned i = threadIdx.x; i < n; i += SBT) {
+        int cc = 0;
+        unsigned base = 0u;
+        for (int q = 0; q < a.S - 1; q++)
+          if (i >= sh.done[q]) {
+            cc = q + 1;
+            base = sh.done[q];
+          }
+        f(i, ld(slabs + (long long)cc * TOPPS_PAIR + (i - base)));
+      }
+    };
+    if (n == 0u) {
+      write_greedy<SBT>(a, r, 0ull);
+    } else {
+      if (n <= (unsigned)CAPL) {
+        each_entry([&](unsigned i, u64 x) { tl.L[i] = x; });
+      } else {
+        // (ties again: the row's top k out of the lists)
+        const u64 T = block_select_kth<u64, 64, SBT>([&](auto f) { each_entry([&](unsigned, u64 x) { f(x); }); },
+                                                     (unsigned)r.k, sh.bs);
+        if (threadIdx.x == 0) sh.ts.ng = 0;
+        __syncthreads();
+        each_entry([&](unsigned, u64 x) {
+          if (x >= T) tl.L[atomicAdd(&sh.ts.ng, 1u)] = x;
+        });
+        n = (unsigned)r.k;
+      }
+      __syncthreads();
+      finish_topk(a, r, tl.L, n, tl, sh);
+    }
+    reset_line(a, cnt, maxima, ep);
+    return;
+  }
+
   // ---- 1. the row's maximum
-  u64 mc = wave_max(thread_best<Tin, SBT>(rv));
+  mc = wave_max(mc);
   if (lane == 0) sh.ts.red64[w] = mc;
   __syncthreads();
+  if (r.mode == 0) {
+    // a greedy row: the last chunk to arrive takes the largest of them all
+    if (w == 0) {
+      mc = wave_max(lane < SBT / 64 ? sh.ts.red64[lane] : 0ull);
+      if (lane == 0) {
+        st(maxima + c, max_entry(mc, ep));
+        wait_stores();
+        sh.arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+    __syncthreads();
+    if (sh.arrived != (unsigned)(a.S - 1)) return;
+    if (w == 0) {
+      const u64 x = wave_max(lane < a.S ? ld(maxima + lane) : 0ull);
+      if (lane == 0) sh.rowmax = max_comp(x);
+    }
+    __syncthreads();
+    write_greedy<SBT>(a, r, sh.rowmax);
+    reset_line(a, cnt, maxima, ep);
+    return;
+  }
   if (w == 0) {
     mc = wave_max(lane < SBT / 64 ? sh.ts.red64[lane] : 0ull);
     if (lane == 0) st(maxima + c, max_entry(mc, ep));
-    const bool act = lane < a.S;
-    u64 e = 0ull;
-    bool ok = false;
-    for (int spins = 0;; spins++) {
-      if (act && !max_current(e, ep)) e = ld(maxima + lane);
-      ok = __ballot(act && !max_current(e, ep)) == 0ull;
-      if (ok || spins >= a.key_spins) break;
-      __builtin_amdgcn_s_sleep(1);
-    }
+    u64 e;
+    const bool ok = poll_words(maxima, a.S, ep, a.key_spins, &e);
     // (entries of the call order as their composites)
-    const u64 x = wave_max(act && ok ? e : 0ull);
+    const u64 x = wave_max(ok ? e : 0ull);
     if (lane == 0) {
-      sh.rowmax = (x >> 32) ? comp_key((uint32_t)(x >> 32), (int)(SIDM - (uint32_t)(x & SIDM))) : 0ull;
+      sh.rowmax = max_comp(x);
       sh.flag = ok;
     }
   }
@@ -213,10 +467,9 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     Mc = block_reduce_max<SBT>(best, sh.ts.red64);
   }
   tl.m = Mc ? comp_y(Mc) : 0.0f;
-  const bool sampling = Mc != 0ull && r.mode == 2;
+  const bool sampling = Mc != 0ull;
 
   // ---- 2. the chunk's histogram, its slab, and the arrival
-  u64* slab = a.ws + ((long long)lb * a.S + c) * TOPPS_PAIR;
   if (sampling) {
     histogram(rv, tl);
     __syncthreads();
@@ -242,12 +495,12 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       int spins = 0;
       for (; spins <= a.key_spins; spins++) {
         d = ld(decision);
-        if ((uint32_t)(d >> 32) == ep) break;
+        if (decided(d, ep)) break;
         __builtin_amdgcn_s_sleep(1);
       }
       if (lane == 0) {
-        sh.flag = (uint32_t)(d >> 32) == ep;
-        sh.word = (uint32_t)d;
+        sh.flag = decided(d, ep);
+        sh.word = d;
         sh.ts.ng = 0;
       }
     }
@@ -256,7 +509,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       if (threadIdx.x == 0) st(done + c, ((u64)ep << 32) | DONE_LEFT);
       return;
     }
-    if (!(sh.word & 1u)) return;  // the owner settles the row by itself
+    if (!(sh.word & 1ull)) return;  // the owner settles the row by itself
     const Plan pl = unpack_plan(sh.word);
     u64* list = slab + TOPPS_SLAB;
     gather(rv, pl, tl.m, sh.ts, [&](int l, unsigned o, u64 x) {
@@ -275,8 +528,8 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   // ---- the owner: the row's histogram, the cut and the draw
   if (!sampling) {
     write_greedy<SBT>(a, r, Mc);
+    if (threadIdx.x == 0) st(decision, (u64)0);
   } else {
-    const u64* slabs = a.ws + (long long)lb * a.S * TOPPS_PAIR;
     {
       // thread t sums buckets t and t + 512, eight slabs' words in flight
       u64 ms[2] = {0ull, 0ull};
@@ -316,12 +569,18 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
     __syncthreads();
     bucket::prefix<SBT>(tl.CI, tl.MI, sh.ts.red32, sh.ts.red64);
-    Plan pl = plan_row<SBT>(r, tl, Mc, tl.CI[NB], sh.ts);
-    if (threadIdx.x == 0)
-      st(decision, ((u64)ep << 32) | pack_plan(pl));
+    const unsigned nall = tl.CI[NB];
+    const unsigned kk = has_k && (unsigned)r.k < nall ? (unsigned)r.k : nall;
+    Plan pl;
+    bool lists = true;
+    if (kk == nall) plan_row<SBT>(pl, r, tl, Mc, nall, sh.ts);
+    else if (kk <= tl.CI[NB - 1]) plan_topk<SBT>(pl, r, tl, Mc, kk, sh.ts);
+    else lists = false;  // the top-k set reaches the mass-0 bucket
+    lists = lists && packs(pl);
+    if (threadIdx.x == 0) st(decision, (u64)(ep & 0xFFFFFFu) << 40 | (lists ? pack_plan(pl) : 0ull));
     SV sv(a, r, hash, hbits, rowp);
     u64 pick;
-    if (packs(pl)) {
+    if (lists) {
       auto take = [&](int l, unsigned o, u64 x) { tl.L[l ? pl.ob + o : o] = x; };
       gather(rv, pl, tl.m, sh.ts, take);
       if (w == 0) {
@@ -384,19 +643,17 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
         }
       }
       __syncthreads();
-      pick = pick_gathered<SBT>(pl, tl, sh.ts, sh.bs);
+      pick = pick_gathered<SBT>(pl, r.top_p, tl, sh.ts, sh.bs);
     } else {
-      pick = pick_resolved<SBT>(pl, sv, tl, sh.ts, sh.bs);
+      if (kk < nall) {
+        pick = pick_streamed<SBT>(pl, kk, r, sv, Mc, tl, sh.ts, sh.bs);
+      } else {
+        pick = pick_resolved<SBT>(pl, sv, tl, sh.ts, sh.bs);
+      }
     }
     write_row<SBT>(a, b, pl, pick, sv, sh.ts);
   }
-  // ready for the next call: counter zero, maxima cleared, epoch advanced
-  // (every workgroup of the row has arrived, so nothing polls the maxima)
-  if (threadIdx.x < (unsigned)a.S) st(maxima + threadIdx.x, (u64)0);
-  if (threadIdx.x == 0) {
-    st(cnt, 0u);
-    st(cnt + 1, ep == 0xFFFFFFFFu ? 0u : ep);
-  }
+  reset_line(a, cnt, maxima, ep);
 }
 
 }  // namespace topp
