@@ -100,9 +100,14 @@ void free_spec(tgs_ctx* h) {
   h->spec_nbs = 0;
 }
 
-// Chunks per row of the fused top_k <= 64 kernel: about one workgroup per CU
-// (chunks of at least 2048 ids), never fewer chunks than a workgroup's
-// capacity requires, at most K64_MAX_SPLIT.  TGS_SPLIT sets the split
+// Chunks per row of the fused top_k <= 64 kernel: as many as keep the launch
+// within one workgroup per CU (chunks of at least 2048 ids), never fewer than
+// a workgroup's capacity requires, at most K64_MAX_SPLIT.  One workgroup more
+// than there are CUs costs a second round or the two-per-CU instantiation:
+// 24 rows of 151,936 fp32 ids took 22.0 us over 11 chunks each (264
+// workgroups) and take 12.3 over 10.  Where the capacity alone forces more
+// workgroups than CUs, more chunks gain nothing: 100 rows of 128,256 take
+// 17.0 us over 4, 17.5 over 5, 25.6 over 6.  TGS_SPLIT sets the split
 // (tuning, tests).
 constexpr int kMaxSplitK64 = tgs::K64_MAX_SPLIT;
 int choose_split_k64(int num_cu, int B, int V, int dt) {
@@ -113,7 +118,7 @@ int choose_split_k64(int num_cu, int B, int V, int dt) {
   if (env && std::atoi(env) > 0) {
     S = std::min(std::atoi(env), kMaxSplitK64);
   } else {
-    S = std::min(kMaxSplitK64, std::max(1, (num_cu + B - 1) / B));
+    S = std::min(kMaxSplitK64, std::max(1, num_cu / B));
     while (S > 1 && (V + S - 1) / S < 2048) S--;
   }
   return std::max(S, smin);
@@ -154,7 +159,7 @@ size_t k64_static() { return tgs::k64_static_lds() + 256; }
 // at once (then its chunks can wait on each other for the row-wide bound),
 // from the runtime's occupancy of the instantiation; cached per variant and
 // LDS size.  TGS_XCHG=0 turns the exchange off (tuning, tests).
-bool k64_resident(int num_cu, int dt, bool whole_vec, bool mask, size_t lds, long long wgs) {
+bool k64_resident(int num_cu, int dt, bool whole_vec, bool mask, size_t lds, bool pair, long long wgs) {
   const char* env = std::getenv("TGS_XCHG");
   if (env && std::atoi(env) == 0) return false;
   struct Entry {
@@ -164,7 +169,7 @@ bool k64_resident(int num_cu, int dt, bool whole_vec, bool mask, size_t lds, lon
   };
   static std::mutex mu;
   static std::vector<Entry> cache;
-  const int key = dt * 4 + (whole_vec ? 2 : 0) + (mask ? 1 : 0);
+  const int key = dt * 8 + (whole_vec ? 4 : 0) + (mask ? 2 : 0) + (pair ? 1 : 0);
   int n = -1;
   {
     std::lock_guard<std::mutex> lock(mu);
@@ -172,7 +177,7 @@ bool k64_resident(int num_cu, int dt, bool whole_vec, bool mask, size_t lds, lon
       if (e.key == key && e.lds == lds) n = e.n;
   }
   if (n < 0) {
-    n = tgs::k64_resident_per_cu(dt, whole_vec, mask, lds);
+    n = tgs::k64_resident_per_cu(dt, whole_vec, mask, lds, pair);
     std::lock_guard<std::mutex> lock(mu);
     cache.push_back({key, lds, n});
   }
@@ -303,8 +308,13 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     // split rows share a row-wide bound when every workgroup of the launch
     // is resident at once: each wave publishes its kq largest thread maxima
     // (at least 64 keys per row, at most K64_KEYS)
+    // more workgroups than CUs: the instantiation that fits two to a CU (64
+    // rows of 151,936 fp32 ids over 5 chunks 23.2 -> 17.1 us, with a mask 25.2
+    // -> 19.9; 512 rows of 128,256 bf16 56 -> 41); up to one per CU the other,
+    // whose registers do not spill (64 masked rows of 128,256: 13.9 against 14.9)
+    const bool pair = (long long)B * a.S > res.num_cu;
     a.xchg = a.S > 1 && k64_resident(res.num_cu, dt, a.whole_vec != 0, res.mask_table != nullptr && res.n_states > 0,
-                                     lds, (long long)B * a.S);
+                                     lds, pair, (long long)B * a.S);
     // keys per wave: the row's S * waves * kq keys fit its K64_KEYS slots
     a.kq = a.S >= 4 ? 4 : 8;
     while (a.kq > 1 && a.S * (tgs::K64_NT / 64) * a.kq > tgs::K64_KEYS) a.kq /= 2;
@@ -332,7 +342,7 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     if (std::getenv("TGS_LOG_LAUNCH"))  // diagnostics: the launch's shape
       std::fprintf(stderr, "tgs k64: B=%d V=%d S=%d L=%d lds=%zu xchg=%d kq=%d xmap=%d small=%d\n", B, V, a.S, a.L,
                    lds, a.xchg, a.kq, a.xmap, (int)small);
-    hipError_t e = tgs::launch_k64(a, dt, lds, stream, small);
+    hipError_t e = tgs::launch_k64(a, dt, lds, stream, small, pair);
     if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
     return TGS_OK;
   }

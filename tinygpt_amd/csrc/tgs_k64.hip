@@ -452,8 +452,8 @@ __device__ __forceinline__ uint4 chunk_vec(const Tin* rowp, int i, int v0, int v
   }
 }
 
-template <typename Tin, int NTT, bool VEC, bool MASK>
-__global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
+template <typename Tin, int NTT, bool VEC, bool MASK, int WPE>
+__global__ __launch_bounds__(NTT, WPE) void k64_kernel(SampleArgs a) {
   using G = Geo<Tin, NTT>;
   constexpr int EPV = G::EPV, NW = G::NW, NHID = G::NHID;
   constexpr uint32_t GM = G::GM;
@@ -547,6 +547,21 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
   r.v0 = v0;
   r.v1 = v1;
   const bool masked = MASK && r.mrow != nullptr;
+  // forbidden-id bits of the thread's vectors (vector i at bit i * EPV),
+  // packed as soon as the words are in (they were requested before most of
+  // the chunk, which streams in behind them): sixteen words held through the
+  // maxima took the kernel past 128 registers, one workgroup per CU
+  constexpr int HPW = HBits<Tin, NTT>::HPW;
+  uint32_t xpk[MASK ? HPW : 1] = {};
+  if constexpr (MASK) {
+    if (masked) {
+#pragma unroll
+      for (int i = 0; i < NVT; i++)
+        xpk[(i * EPV) >> 5] |= (~(mw[i] >> ((v0 + ((int)threadIdx.x + i * NTT) * EPV) & 31)) & GM) << ((i * EPV) & 31);
+    }
+#pragma unroll
+    for (int q = 0; q < HPW; q++) asm volatile("" : "+v"(xpk[q]));  // keep the packing here
+  }
 
   // ---- history, first its bits: each id of the chunk marked in the packed
   // history bits (HBits), all the bound needs.  The id -> count table is
@@ -558,7 +573,6 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
   }
   const bool pen = r.use_pen;
   using HB = HBits<Tin, NTT>;
-  constexpr int HPW = HB::HPW;
   if (pen) {
     for (int i = threadIdx.x; i < a.TS; i += NTT) hash[i] = make_int2(-1, 0);
 #pragma unroll
@@ -621,20 +635,18 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
   float vm[NVT];
   float tm = -__builtin_inff();
   int im = 0;
-  uint32_t xpk[MASK ? HPW : 1] = {};  // forbidden-id bits of the thread's vectors (vector i at bit i * EPV)
 #pragma unroll
   for (int i = 0; i < NVT; i++) {
     float m;
     if constexpr (MASK) {
       // an id the mask forbids becomes a quiet NaN (its bits ORed with
-      // 0xFFC00000, through the sign-extended bit of x), which the maximum
+      // 0xFFC00000, through its sign-extended bit), which the maximum
       // ignores: two operations per id instead of a test and a select
-      const uint32_t x = masked ? ~(mw[i] >> ((v0 + ((int)threadIdx.x + i * NTT) * EPV) & 31)) : 0u;
-      xpk[(i * EPV) >> 5] |= (x & GM) << ((i * EPV) & 31);
       m = -__builtin_inff();
 #pragma unroll
       for (int e = 0; e < EPV; e++) {
-        const uint32_t off = (uint32_t)((int)(x << (31 - e)) >> 31) & 0xFFC00000u;
+        const int bit = i * EPV + e;
+        const uint32_t off = (uint32_t)((int)(xpk[bit >> 5] << (31 - (bit & 31))) >> 31) & 0xFFC00000u;
         m = fmaxf(m, tg_u2f(tg_f2u(Elem<Tin>::get(raw[i], e)) | off));
       }
     } else {
@@ -670,7 +682,7 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
         if (i * NTT >= nvec) break;  // (uniform) no thread holds vector i
         const bool live = i < nfull || (int)threadIdx.x + i * NTT < nvec;
         uint32_t x = 0u;
-        if constexpr (MASK) x = masked ? ~(mw[i] >> ((v0 + ((int)threadIdx.x + i * NTT) * EPV) & 31)) & GM : 0u;
+        if constexpr (MASK) x = (xpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
 #pragma unroll
         for (int e = 0; e < EPV; e++) {
           const int bit = i * EPV + e;
@@ -806,7 +818,7 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
         const bool pass = ((pm >> i) & 1u) && j < nvec;
         const uint32_t hw = (hpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
         uint32_t xm = 0u;
-        if constexpr (MASK) xm = masked ? ~(mw[i] >> ((v0 + o) & 31)) & GM : 0u;
+        if constexpr (MASK) xm = (xpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
         u64 x[EPV];
         bool ok[EPV];
 #pragma unroll
@@ -1056,44 +1068,48 @@ __global__ __launch_bounds__(NTT) void k64_kernel(SampleArgs a) {
   }
 }
 
-template <typename Tin, int NTT>
+// The K64_NT instantiations come in two register budgets: as many as the
+// compiler likes (134 - 154: one workgroup per CU) for launches of at most
+// one workgroup per CU, and at most 128 (WPE = 4 waves per SIMD: two
+// workgroups per CU) for larger ones.
+template <typename Tin, int NTT, int WPE>
+const void* kernel_of(bool vec, bool mask) {
+  return vec && mask ? (const void*)k64_kernel<Tin, NTT, true, true, WPE>
+         : vec       ? (const void*)k64_kernel<Tin, NTT, true, false, WPE>
+         : mask      ? (const void*)k64_kernel<Tin, NTT, false, true, WPE>
+                     : (const void*)k64_kernel<Tin, NTT, false, false, WPE>;
+}
+
+template <typename Tin, int NTT, int WPE>
 hipError_t launch_n(const SampleArgs& a, size_t lds, hipStream_t st) {
   const dim3 g(a.B * a.S), blk(NTT);
   const bool vec = a.whole_vec != 0, mask = a.mask_table != nullptr && a.n_states > 0;
-  if (vec && mask) hipLaunchKernelGGL((k64_kernel<Tin, NTT, true, true>), g, blk, lds, st, a);
-  else if (vec) hipLaunchKernelGGL((k64_kernel<Tin, NTT, true, false>), g, blk, lds, st, a);
-  else if (mask) hipLaunchKernelGGL((k64_kernel<Tin, NTT, false, true>), g, blk, lds, st, a);
-  else hipLaunchKernelGGL((k64_kernel<Tin, NTT, false, false>), g, blk, lds, st, a);
+  if (vec && mask) hipLaunchKernelGGL((k64_kernel<Tin, NTT, true, true, WPE>), g, blk, lds, st, a);
+  else if (vec) hipLaunchKernelGGL((k64_kernel<Tin, NTT, true, false, WPE>), g, blk, lds, st, a);
+  else if (mask) hipLaunchKernelGGL((k64_kernel<Tin, NTT, false, true, WPE>), g, blk, lds, st, a);
+  else hipLaunchKernelGGL((k64_kernel<Tin, NTT, false, false, WPE>), g, blk, lds, st, a);
   return hipGetLastError();
 }
 
 // Workgroups of the K64_NT instantiation one CU holds at once with lds bytes
 // of dynamic LDS (0 when the runtime cannot say).
-template <typename Tin>
+template <typename Tin, int WPE>
 int resident_n(bool vec, bool mask, size_t lds) {
-  const void* f = vec && mask ? (const void*)k64_kernel<Tin, K64_NT, true, true>
-                  : vec       ? (const void*)k64_kernel<Tin, K64_NT, true, false>
-                  : mask      ? (const void*)k64_kernel<Tin, K64_NT, false, true>
-                              : (const void*)k64_kernel<Tin, K64_NT, false, false>;
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, K64_NT, lds) != hipSuccess) {
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel_of<Tin, K64_NT, WPE>(vec, mask), K64_NT, lds) !=
+      hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
   return n;
 }
 
-template <typename Tin, int NTT>
+template <typename Tin, int NTT, int WPE>
 hipError_t set_lds(size_t bytes) {
-  const void* fns[] = {
-      (const void*)k64_kernel<Tin, NTT, true, true>,
-      (const void*)k64_kernel<Tin, NTT, true, false>,
-      (const void*)k64_kernel<Tin, NTT, false, true>,
-      (const void*)k64_kernel<Tin, NTT, false, false>,
-  };
   hipError_t e = hipSuccess;
-  for (const void* f : fns) {
-    hipError_t e2 = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+  for (int i = 0; i < 4; i++) {
+    hipError_t e2 = hipFuncSetAttribute(kernel_of<Tin, NTT, WPE>((i & 1) != 0, (i & 2) != 0),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e2 != hipSuccess) e = e2;
   }
   return e;
@@ -1107,22 +1123,27 @@ int k64_small_ids(int dtype) { return K64_SMALL_NT * K64_NVT * (dtype == 1 ? 8 :
 
 size_t k64_static_lds() { return sizeof(k64::Shared<K64_NT / 64>); }
 
-int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds) {
-  return dtype == 1 ? k64::resident_n<uint16_t>(whole_vec, mask, lds) : k64::resident_n<float>(whole_vec, mask, lds);
+int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds, bool pair) {
+  if (pair)
+    return dtype == 1 ? k64::resident_n<uint16_t, 4>(whole_vec, mask, lds) : k64::resident_n<float, 4>(whole_vec, mask, lds);
+  return dtype == 1 ? k64::resident_n<uint16_t, 1>(whole_vec, mask, lds) : k64::resident_n<float, 1>(whole_vec, mask, lds);
 }
 
-hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small) {
+hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small, bool pair) {
   if (small)
-    return dtype == 1 ? k64::launch_n<uint16_t, K64_SMALL_NT>(a, lds, st) : k64::launch_n<float, K64_SMALL_NT>(a, lds, st);
-  return dtype == 1 ? k64::launch_n<uint16_t, K64_NT>(a, lds, st) : k64::launch_n<float, K64_NT>(a, lds, st);
+    return dtype == 1 ? k64::launch_n<uint16_t, K64_SMALL_NT, 1>(a, lds, st)
+                      : k64::launch_n<float, K64_SMALL_NT, 1>(a, lds, st);
+  if (pair)
+    return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 4>(a, lds, st) : k64::launch_n<float, K64_NT, 4>(a, lds, st);
+  return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 1>(a, lds, st) : k64::launch_n<float, K64_NT, 1>(a, lds, st);
 }
 
 hipError_t set_k64_lds_limit(size_t bytes) {
-  hipError_t e = hipSuccess, e2;
-  if ((e2 = k64::set_lds<float, K64_NT>(bytes)) != hipSuccess) e = e2;
-  if ((e2 = k64::set_lds<uint16_t, K64_NT>(bytes)) != hipSuccess) e = e2;
-  if ((e2 = k64::set_lds<float, K64_SMALL_NT>(bytes)) != hipSuccess) e = e2;
-  if ((e2 = k64::set_lds<uint16_t, K64_SMALL_NT>(bytes)) != hipSuccess) e = e2;
+  hipError_t e = hipSuccess;
+  for (const hipError_t e2 : {k64::set_lds<float, K64_NT, 1>(bytes), k64::set_lds<uint16_t, K64_NT, 1>(bytes),
+                              k64::set_lds<float, K64_NT, 4>(bytes), k64::set_lds<uint16_t, K64_NT, 4>(bytes),
+                              k64::set_lds<float, K64_SMALL_NT, 1>(bytes), k64::set_lds<uint16_t, K64_SMALL_NT, 1>(bytes)})
+    if (e2 != hipSuccess) e = e2;
   return e;
 }
 

@@ -178,10 +178,11 @@ int k64_chunk_ids(int dtype);
 // small: the one-wave variant (K64_SMALL_NT threads, one chunk per row of at
 // most k64_small_ids(dtype) ids, history <= K64_SMALL_MAX_HIST).
 int k64_small_ids(int dtype);
-hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small = false);
+// pair: the instantiation of which two workgroups fit a CU.
+hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small, bool pair);
 // Workgroups of the K64_NT instantiation that one CU holds at once with lds
 // bytes of dynamic LDS (0 when the runtime cannot tell).
-int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds);
+int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds, bool pair);
 // Static LDS of the K64_NT instantiation.
 size_t k64_static_lds();
 hipError_t set_k64_lds_limit(size_t bytes);
