@@ -342,7 +342,12 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     if (std::getenv("TGS_LOG_LAUNCH"))  // diagnostics: the launch's shape
       std::fprintf(stderr, "tgs k64: B=%d V=%d S=%d L=%d lds=%zu xchg=%d kq=%d xmap=%d small=%d\n", B, V, a.S, a.L,
                    lds, a.xchg, a.kq, a.xmap, (int)small);
-    hipError_t e = tgs::launch_k64(a, dt, lds, stream, small, pair);
+    const bool mid = pair && a.S == 1 && V <= tgs::k64_mid_ids(dt);
+    hipError_t e = tgs::launch_k64(a, dt, lds, stream,
+                                   small  ? tgs::K64Kind::small
+                                   : mid  ? tgs::K64Kind::mid
+                                   : pair ? tgs::K64Kind::pair
+                                          : tgs::K64Kind::single);
     if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
     return TGS_OK;
   }

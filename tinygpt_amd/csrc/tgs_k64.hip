@@ -34,8 +34,8 @@
 //      A wave collects from cz, 16 representable values below its bound
 //      (the larger of the two).
 //   3. Every vector whose maximum reaches cz is staged whole in its wave's
-//      LDS list (a one-wave row of at most two vectors per thread skips the
-//      staging: each lane tests its own vectors in step 4).
+//      LDS list (a one-wave row, of at most two vectors per thread, skips
+//      the staging: each lane tests its own vectors in step 4).
 //   4. One staged vector per lane: every allowed element whose raw logit z
 //      reaches cz becomes a composite of z and its id, history ids left to
 //      their producers (the lane whose insertion created the id's LDS hash
@@ -84,7 +84,6 @@
 namespace tgs {
 namespace k64 {
 
-constexpr int NVT = K64_NVT;         // 16-byte vectors per thread
 constexpr int KM = 64;               // largest top_k served; longest published list
 constexpr int CAP = K64_CAP;         // candidate buffer entries
 constexpr u64 EMPTY = 0ull;          // list entry not written: a published entry never is 0
@@ -96,8 +95,9 @@ template <typename Tin, int NTT>
 struct Geo {
   static constexpr int EPV = Elem<Tin>::EPV;
   static constexpr int NW = NTT / 64;
+  static constexpr int NVT = NTT >= K64_NT ? K64_NVT : NTT >= K64_MID_NT ? K64_MID_NVT : K64_SMALL_NVT;  // 16-byte vectors per thread
   static constexpr int CH = NTT * NVT * EPV;  // ids of a chunk at most
-  static constexpr int MAXH = NTT >= K64_NT ? K64_MAX_HIST : K64_SMALL_MAX_HIST;  // longest history
+  static constexpr int MAXH = NTT >= K64_MID_NT ? K64_MAX_HIST : K64_SMALL_MAX_HIST;  // longest history
   static constexpr int NHID = (MAXH + NTT - 1) / NTT;  // history ids per thread (its share of the row's)
   static constexpr uint32_t GM = (1u << EPV) - 1u;
 };
@@ -128,7 +128,7 @@ struct Shared {
 template <typename Tin, int NTT>
 struct HBits {
   static constexpr int EPV = Elem<Tin>::EPV;
-  static constexpr int HPW = NVT * EPV / 32;  // words per thread
+  static constexpr int HPW = (Geo<Tin, NTT>::NVT * EPV + 31) / 32;  // words per thread
   static constexpr int WORDS = NTT * HPW;
   static constexpr uint32_t GM = (1u << EPV) - 1u;
   __device__ static int word(int j) { return (j % NTT) * HPW + (j / NTT) * EPV / 32; }
@@ -455,7 +455,7 @@ __device__ __forceinline__ uint4 chunk_vec(const Tin* rowp, int i, int v0, int v
 template <typename Tin, int NTT, bool VEC, bool MASK, int WPE>
 __global__ __launch_bounds__(NTT, WPE) void k64_kernel(SampleArgs a) {
   using G = Geo<Tin, NTT>;
-  constexpr int EPV = G::EPV, NW = G::NW, NHID = G::NHID;
+  constexpr int EPV = G::EPV, NW = G::NW, NHID = G::NHID, NVT = G::NVT;
   constexpr uint32_t GM = G::GM;
   constexpr int SCAP = 64;   // staged vectors per wave
   TGS_DYN_SMEM(smem);
@@ -612,7 +612,9 @@ __global__ __launch_bounds__(NTT, WPE) void k64_kernel(SampleArgs a) {
   // load while the chunk is still in flight
   uint32_t hpk[HPW];
   if (pen) {
-    if constexpr (HPW == 2) {
+    if constexpr (HPW == 1) {
+      hpk[0] = bitmap[threadIdx.x];
+    } else if constexpr (HPW == 2) {
       const uint2 t = *(const uint2*)(bitmap + threadIdx.x * HPW);
       hpk[0] = t.x;
       hpk[1] = t.y;
@@ -805,33 +807,28 @@ __global__ __launch_bounds__(NTT, WPE) void k64_kernel(SampleArgs a) {
   for (int i = 0; i < NVT; i++)
     pm |= (vm[i] >= cz && vm[i] > -__builtin_inff()) ? (1u << i) : 0u;  // (cz may be -inf)
   const uint32_t PM = wave_or(pm);
-  bool direct = false;  // (uniform)
   if constexpr (NTT == 64) {
-    // one wave over at most two vectors per thread: each lane tests its own
-    // vectors from its registers (no staging round trip through LDS)
-    if (nvec <= 2 * NTT) {
-      direct = true;
+    // one wave: each lane tests its own vectors from its registers (no
+    // staging round trip through LDS)
 #pragma unroll
-      for (int i = 0; i < 2; i++) {
-        if (!(PM & (1u << i))) continue;  // uniform
-        const int j = (int)threadIdx.x + i * NTT, o = j * EPV;
-        const bool pass = ((pm >> i) & 1u) && j < nvec;
-        const uint32_t hw = (hpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
-        uint32_t xm = 0u;
-        if constexpr (MASK) xm = (xpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
-        u64 x[EPV];
-        bool ok[EPV];
+    for (int i = 0; i < NVT; i++) {
+      if (!(PM & (1u << i))) continue;  // uniform
+      const int j = (int)threadIdx.x + i * NTT, o = j * EPV;
+      const bool pass = ((pm >> i) & 1u) && j < nvec;
+      const uint32_t hw = (hpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
+      uint32_t xm = 0u;
+      if constexpr (MASK) xm = (xpk[(i * EPV) >> 5] >> ((i * EPV) & 31)) & GM;
+      u64 x[EPV];
+      bool ok[EPV];
 #pragma unroll
-        for (int e = 0; e < EPV; e++) {
-          const float z = Elem<Tin>::get(raw[i], e);
-          ok[e] = pass && z >= cz && z > -__builtin_inff() && !((hw >> e) & 1u) && !((xm >> e) & 1u);
-          x[e] = comp_key(tg_key(z), v0 + o + e);
-        }
-        append_n<EPV>(x, ok, buf, &sh.nbuf);
+      for (int e = 0; e < EPV; e++) {
+        const float z = Elem<Tin>::get(raw[i], e);
+        ok[e] = pass && z >= cz && z > -__builtin_inff() && !((hw >> e) & 1u) && !((xm >> e) & 1u);
+        x[e] = comp_key(tg_key(z), v0 + o + e);
       }
+      append_n<EPV>(x, ok, buf, &sh.nbuf);
     }
-  }
-  if (!direct) {
+  } else {
     unsigned ns = 0;  // staged vectors of the wave (uniform)
 #pragma unroll
     for (int i = 0; i < NVT; i++) {
@@ -1119,7 +1116,7 @@ hipError_t set_lds(size_t bytes) {
 
 int k64_chunk_ids(int dtype) { return K64_NT * K64_NVT * (dtype == 1 ? 8 : 4); }
 
-int k64_small_ids(int dtype) { return K64_SMALL_NT * K64_NVT * (dtype == 1 ? 8 : 4); }
+int k64_small_ids(int dtype) { return K64_SMALL_NT * K64_SMALL_NVT * (dtype == 1 ? 8 : 4); }
 
 size_t k64_static_lds() { return sizeof(k64::Shared<K64_NT / 64>); }
 
@@ -1129,19 +1126,28 @@ int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds, bool p
   return dtype == 1 ? k64::resident_n<uint16_t, 1>(whole_vec, mask, lds) : k64::resident_n<float, 1>(whole_vec, mask, lds);
 }
 
-hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small, bool pair) {
-  if (small)
-    return dtype == 1 ? k64::launch_n<uint16_t, K64_SMALL_NT, 1>(a, lds, st)
-                      : k64::launch_n<float, K64_SMALL_NT, 1>(a, lds, st);
-  if (pair)
-    return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 4>(a, lds, st) : k64::launch_n<float, K64_NT, 4>(a, lds, st);
-  return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 1>(a, lds, st) : k64::launch_n<float, K64_NT, 1>(a, lds, st);
+int k64_mid_ids(int dtype) { return K64_MID_NT * K64_MID_NVT * (dtype == 1 ? 8 : 4); }
+
+hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, K64Kind kind) {
+  switch (kind) {
+    case K64Kind::small:
+      return dtype == 1 ? k64::launch_n<uint16_t, K64_SMALL_NT, 1>(a, lds, st)
+                        : k64::launch_n<float, K64_SMALL_NT, 1>(a, lds, st);
+    case K64Kind::mid:
+      return dtype == 1 ? k64::launch_n<uint16_t, K64_MID_NT, 4>(a, lds, st)
+                        : k64::launch_n<float, K64_MID_NT, 4>(a, lds, st);
+    case K64Kind::pair:
+      return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 4>(a, lds, st) : k64::launch_n<float, K64_NT, 4>(a, lds, st);
+    default:
+      return dtype == 1 ? k64::launch_n<uint16_t, K64_NT, 1>(a, lds, st) : k64::launch_n<float, K64_NT, 1>(a, lds, st);
+  }
 }
 
 hipError_t set_k64_lds_limit(size_t bytes) {
   hipError_t e = hipSuccess;
   for (const hipError_t e2 : {k64::set_lds<float, K64_NT, 1>(bytes), k64::set_lds<uint16_t, K64_NT, 1>(bytes),
                               k64::set_lds<float, K64_NT, 4>(bytes), k64::set_lds<uint16_t, K64_NT, 4>(bytes),
+                              k64::set_lds<float, K64_MID_NT, 4>(bytes), k64::set_lds<uint16_t, K64_MID_NT, 4>(bytes),
                               k64::set_lds<float, K64_SMALL_NT, 1>(bytes), k64::set_lds<uint16_t, K64_SMALL_NT, 1>(bytes)})
     if (e2 != hipSuccess) e = e2;
   return e;

@@ -19,7 +19,17 @@ constexpr int K64_NT = 512;
 constexpr int K64_NVT = 16;
 constexpr int K64_MASK_PRE = 2;  // with a mask table: chunk vectors requested before the mask words
 constexpr int K64_MAX_HIST = 1024;
-constexpr int K64_SMALL_NT = 64;        // one-wave variant for rows of one small chunk
+// One-wave variant for rows of one small chunk, at most two vectors per
+// thread (64 rows of 512 fp32 ids 13.0 us against 13.4 with eight waves, 1000
+// rows 13.0 against 25.7; with more vectors a wave's serial collection costs
+// more than seven idle waves: 64 rows of 768 19.1 against 13.4, of 4096 56
+// against 13.5).
+constexpr int K64_SMALL_NT = 64;
+constexpr int K64_SMALL_NVT = 2;
+// Four-wave variant for more rows than CUs that fit one chunk of eight
+// vectors per thread: four workgroups per CU instead of two.
+constexpr int K64_MID_NT = 256;
+constexpr int K64_MID_NVT = 8;
 constexpr int K64_SMALL_MAX_HIST = 256;  // its longest history
 constexpr int K64_CAP = 2048;
 constexpr int K64_MAX_SPLIT = 16;
@@ -178,8 +188,11 @@ int k64_chunk_ids(int dtype);
 // small: the one-wave variant (K64_SMALL_NT threads, one chunk per row of at
 // most k64_small_ids(dtype) ids, history <= K64_SMALL_MAX_HIST).
 int k64_small_ids(int dtype);
-// pair: the instantiation of which two workgroups fit a CU.
-hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, bool small, bool pair);
+// mid: K64_MID_NT threads, one chunk per row of at most k64_mid_ids(dtype)
+// ids.  pair: the K64_NT instantiation of which two workgroups fit a CU.
+int k64_mid_ids(int dtype);
+enum class K64Kind { small, mid, pair, single };
+hipError_t launch_k64(const SampleArgs& a, int dtype, size_t lds, hipStream_t st, K64Kind kind);
 // Workgroups of the K64_NT instantiation that one CU holds at once with lds
 // bytes of dynamic LDS (0 when the runtime cannot tell).
 int k64_resident_per_cu(int dtype, bool whole_vec, bool mask, size_t lds, bool pair);
