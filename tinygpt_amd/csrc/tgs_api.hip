@@ -540,11 +540,14 @@ int tgs_create(tgs_handle* out, int device, int max_batch, int max_vocab, int ma
   if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && v > 0)
     h->lds_limit = (size_t)v;
   h->ws_rows = std::max(max_batch, 4 * h->num_cu);
-  // (and room for the split top-p kernel's slabs of 1024 chunks at a time)
-  h->ws_words = std::max((size_t)h->ws_rows * tgs::KMAX,
-                         max_vocab > tgs::topp_resident_ids()
-                             ? (size_t)std::min(1024, max_batch * tgs::TOPPS_MAX_SPLIT) * tgs::TOPPS_PAIR
-                             : (size_t)0);
+  // (and room for the slabs of the split top-p kernel's chunks, at most 1024 at a time)
+  size_t pairs = 0;
+  if (max_vocab > tgs::topp_resident_ids()) {
+    const int smin = (max_vocab + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
+    pairs = std::max((size_t)std::min(h->num_cu, max_batch * tgs::TOPPS_MAX_SPLIT), (size_t)max_batch * smin);
+    pairs = std::min(pairs, (size_t)1024);
+  }
+  h->ws_words = std::max((size_t)h->ws_rows * tgs::KMAX, pairs * tgs::TOPPS_PAIR);
   hipError_t e = hipMalloc(&h->ws, sizeof(unsigned long long) * h->ws_words);
   if (e == hipSuccess) e = hipMalloc(&h->ws_cnt, sizeof(int) * (size_t)h->ws_rows * (tgs::KMAX / 64));
   // everything that starts zeroed in one allocation: chunk lists ("not
