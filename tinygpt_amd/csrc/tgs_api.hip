@@ -831,7 +831,6 @@ int tgs_token_logprobs(tgs_handle h, const void* d_logits, tgs_dtype dt, int B, 
   if (!d_logits || !d_tokens || !d_out_logprob) return fail(h, TGS_EINVAL, "null buffer");
   DeviceGuard g(h->device);
   if (!g.ok) return fail(h, TGS_EHIP, "hipSetDevice");
-  const size_t esz = dt == TGS_BF16 ? 2 : 4;
   const int epv = dt == TGS_BF16 ? 8 : 4;
   tgs::LogprobArgs a;
   std::memset(&a, 0, sizeof(a));
@@ -839,7 +838,6 @@ int tgs_token_logprobs(tgs_handle h, const void* d_logits, tgs_dtype dt, int B, 
   a.row_stride = row_stride;
   a.B = B;
   a.V = V;
-  a.aligned = ((uintptr_t)d_logits % 16 == 0) && (((uint64_t)row_stride * esz) % 16 == 0);
   a.tokens = d_tokens;
   a.out_lp = d_out_logprob;
   a.out_lse = d_out_lse;
@@ -906,7 +904,6 @@ int tgs_spec_verify(tgs_handle h, const void* d_target, const void* d_draft, tgs
   }
   DeviceGuard g(h->device);
   if (!g.ok) return fail(h, TGS_EHIP, "hipSetDevice");
-  const size_t esz = dt == TGS_BF16 ? 2 : 4;
   tgs::SpecArgs a;
   std::memset(&a, 0, sizeof(a));
   a.target = d_target;
@@ -914,7 +911,6 @@ int tgs_spec_verify(tgs_handle h, const void* d_target, const void* d_draft, tgs
   a.B = B;
   a.k = k;
   a.V = V;
-  a.aligned = ((uintptr_t)d_target % 16 == 0) && ((uintptr_t)d_draft % 16 == 0) && (((uint64_t)V * esz) % 16 == 0);
   a.dtok = d_draft_tok;
   a.T = d_T;
   a.u_acc = d_u_acc;

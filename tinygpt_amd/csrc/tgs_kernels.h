@@ -145,7 +145,6 @@ struct LogprobArgs {
   const void* logits;
   long long row_stride;  // elements
   int B, V;
-  int aligned;           // rows start 16-byte aligned: vector loads
   const int* tokens;     // [B]
   float* out_lp;         // [B]
   float* out_lse;        // [B] or nullptr
@@ -158,7 +157,6 @@ struct SpecArgs {
   const void* target;
   const void* draft;
   int B, k, V;
-  int aligned;
   const int* dtok;
   const float* T;
   const float* u_acc;

@@ -3,7 +3,10 @@
 // x[tok] - logsumexp(x)), for B rows.
 //
 // HBM-bound: one read of every logit, 2 or 4 bytes, against about six VALU
-// operations.  Workgroups of 256 threads stream 16-byte vectors (four issued
+// operations.  Rows start at any element alignment (an odd vocabulary): the
+// 16-byte loads take them as they are, in global memory's unaligned access
+// mode, instead of one element per load (2048 rows of 50,257 bf16 125 us, 512
+// of 50,257 fp32 63).  Workgroups of 256 threads stream 16-byte vectors (four issued
 // per thread before any is used) and keep an online pair (m, s): the running
 // maximum and sum of exp(x - m), rescaled when m grows; exp is exp2 of
 // x * log2(e) - m * log2(e) (one fused multiply-add and one v_exp_f32).
@@ -92,14 +95,13 @@ __global__ __launch_bounds__(LT) void chunk_kernel(LogprobArgs a) {
   const int v0 = c * a.L;
   const int v1 = v0 + a.L < a.V ? v0 + a.L : a.V;
   Pair p{-__builtin_inff(), 0.0f};
-  // whole vectors: [v0, vend) when rows are 16-byte aligned, else none
-  const int vend = a.aligned ? v0 + (v1 - v0) / EPV * EPV : v0;
-  const int nvec = (vend - v0) / EPV;
+  const int nvec = (v1 - v0) / EPV;  // whole vectors, at whatever alignment the row starts
+  const int vend = v0 + nvec * EPV;
   int i = threadIdx.x;
   for (; i + (UNR - 1) * LT < nvec; i += UNR * LT) {
     uint4 raw[UNR];
 #pragma unroll
-    for (int u = 0; u < UNR; u++) raw[u] = tg_load_nt(rowp + v0 + (i + u * LT) * EPV);
+    for (int u = 0; u < UNR; u++) raw[u] = load_row16<true>(rowp + v0 + (i + u * LT) * EPV);
     float x[UNR * EPV];
 #pragma unroll
     for (int u = 0; u < UNR; u++)
@@ -108,13 +110,13 @@ __global__ __launch_bounds__(LT) void chunk_kernel(LogprobArgs a) {
     accumulate(p, x);
   }
   for (; i < nvec; i += LT) {
-    const uint4 raw = tg_load_nt(rowp + v0 + i * EPV);
+    const uint4 raw = load_row16<true>(rowp + v0 + i * EPV);
     float x[EPV];
 #pragma unroll
     for (int e = 0; e < EPV; e++) x[e] = Elem<Tin>::get(raw, e);
     accumulate(p, x);
   }
-  for (int v = vend + (int)threadIdx.x; v < v1; v += LT) {  // unaligned rows, the row's tail
+  for (int v = vend + (int)threadIdx.x; v < v1; v += LT) {  // the row's tail
     float x[1] = {Elem<Tin>::scalar(rowp, v)};
     accumulate(p, x);
   }

@@ -65,19 +65,18 @@ __device__ __forceinline__ const Tin* row_ptr(const SpecArgs& a, int b, int r) {
   return (const Tin*)a.draft + ((long long)b * k + (r - k - 1)) * a.V;
 }
 
-// A block wholly inside the row of an aligned row (every block but a row's
-// last when V is not a multiple of the block) takes plain 16-byte loads
-// behind one wave-uniform test; the others test each vector.
+// A block wholly inside the row (every block but a row's last when V is not a
+// multiple of the block) takes plain 16-byte loads, at whatever alignment the
+// row starts, behind one wave-uniform test; the others test each vector.
 template <typename Tin>
-__device__ __forceinline__ void load_block(const Tin* rowp, int blk, int V, bool aligned,
-                                           uint4 (&raw)[Tile<Tin>::NV]) {
-  if (aligned && (blk + 1) * SPEC_BLOCK <= V) {
+__device__ __forceinline__ void load_block(const Tin* rowp, int blk, int V, uint4 (&raw)[Tile<Tin>::NV]) {
+  if ((blk + 1) * SPEC_BLOCK <= V) {
 #pragma unroll
-    for (int i = 0; i < Tile<Tin>::NV; i++) raw[i] = *(const uint4*)(rowp + blk_id<Tin>(blk, i, 0));
+    for (int i = 0; i < Tile<Tin>::NV; i++) raw[i] = load_row16<false>(rowp + blk_id<Tin>(blk, i, 0));
     return;
   }
 #pragma unroll
-  for (int i = 0; i < Tile<Tin>::NV; i++) raw[i] = load_vec<Tin>(rowp, blk_id<Tin>(blk, i, 0), V, aligned);
+  for (int i = 0; i < Tile<Tin>::NV; i++) raw[i] = load_vec<Tin>(rowp, blk_id<Tin>(blk, i, 0), V, false);
 }
 
 // Sequence temperature: greedy (T <= 0), the clamped T = max(T, 1e-5), its
@@ -280,14 +279,14 @@ __global__ __launch_bounds__(NT) void spec_block_kernel(SpecArgs a) {
   pend.m = 0.0f;
   pend.o = -1;
   uint4 cur[TL::NV];
-  if (x.live) load_block<Tin>(row_ptr<Tin>(a, x.b, x.r), x.blk, a.V, a.aligned, cur);
+  if (x.live) load_block<Tin>(row_ptr<Tin>(a, x.b, x.r), x.blk, a.V, cur);
   for (int i = 0; i < n; i++) {
     const bool more = i + 1 < n;
     BlockRef xn = x;
     uint4 nxt[TL::NV];
     if (more) {
       xn = block_next(a, x);
-      if (xn.live) load_block<Tin>(row_ptr<Tin>(a, xn.b, xn.r), xn.blk, a.V, a.aligned, nxt);
+      if (xn.live) load_block<Tin>(row_ptr<Tin>(a, xn.b, xn.r), xn.blk, a.V, nxt);
     }
     if (x.live) block_stats<Tin>(a, x, cur, pend);
     if (!more) break;
@@ -570,8 +569,8 @@ __global__ __launch_bounds__(NT) void spec_mass_kernel(SpecArgs a) {
   if (s.status > 1) return;
   const DrawRow<Tin> dw = draw_row<Tin>(a, b, s, s.status == 1);
   uint4 rt[TL::NV], rd[TL::NV];
-  load_block<Tin>(dw.tr, blk, dw.V, a.aligned, rt);
-  if (dw.resid) load_block<Tin>(dw.dr, blk, dw.V, a.aligned, rd);
+  load_block<Tin>(dw.tr, blk, dw.V, rt);
+  if (dw.resid) load_block<Tin>(dw.dr, blk, dw.V, rd);
   u64* gw = a.blk_w + ((long long)b * a.nbs + blk) * SPEC_GROUPS;
   u64 gq[TL::NV];
 #pragma unroll
@@ -644,8 +643,8 @@ __device__ __forceinline__ int pick_in_group(const SpecArgs& a, const DrawRow<Ti
                                              u64 run) {
   constexpr int EPV = Elem<Tin>::EPV;
   const int v = blk_id<Tin>(blk, i, 0);
-  const uint4 rt = load_vec<Tin>(dw.tr, v, dw.V, a.aligned);
-  const uint4 rd = dw.resid ? load_vec<Tin>(dw.dr, v, dw.V, a.aligned) : rt;
+  const uint4 rt = load_vec<Tin>(dw.tr, v, dw.V, false);
+  const uint4 rd = dw.resid ? load_vec<Tin>(dw.dr, v, dw.V, false) : rt;
   double ws[EPV];
   group_masses<Tin>(dw, rt, rd, ws);
   u64 ls = 0;
@@ -673,8 +672,8 @@ __device__ __forceinline__ int pick_in_block(const SpecArgs& a, const DrawRow<Ti
     // mass of the group, for the next one
     constexpr int EPV = Elem<Tin>::EPV;
     const int v = blk_id<Tin>(blk, i, 0);
-    const uint4 rt = load_vec<Tin>(dw.tr, v, dw.V, a.aligned);
-    const uint4 rd = dw.resid ? load_vec<Tin>(dw.dr, v, dw.V, a.aligned) : rt;
+    const uint4 rt = load_vec<Tin>(dw.tr, v, dw.V, false);
+    const uint4 rd = dw.resid ? load_vec<Tin>(dw.dr, v, dw.V, false) : rt;
     double ws[EPV];
     group_masses<Tin>(dw, rt, rd, ws);
     double ls = 0.0;
@@ -713,7 +712,7 @@ __global__ __launch_bounds__(NT) void spec_draw_kernel(SpecArgs a) {
     const DrawRow<Tin> dw = draw_row<Tin>(a, b, s, false);
     for (int blk = w; blk < a.nb; blk += WPB) {
       uint4 rt[TL::NV];
-      load_block<Tin>(dw.tr, blk, dw.V, a.aligned, rt);
+      load_block<Tin>(dw.tr, blk, dw.V, rt);
       double ls = 0.0;
 #pragma unroll
       for (int i = 0; i < TL::NV; i++) {
