@@ -28,7 +28,7 @@ static std::vector<char> slurp(const std::string& path) {
 }
 static void dump(const std::string& path, const void* p, size_t n) {
   FILE* f = std::fopen(path.c_str(), "wb");
-  std::fwrite(p, 1, n, f);
+  if (n) std::fwrite(p, 1, n, f);
   std::fclose(f);
 }
 

@@ -166,3 +166,58 @@ def test_topk_rows(sampler, oracle, V, bf16, mask, hist):
     np.testing.assert_array_equal(got["mass"].cpu().numpy().view(np.uint64)[ok],
                                   np.stack([o["res"]["mass_k"], o["res"]["mass_p"]], 1)[ok])
     np.testing.assert_array_equal(got["cut_ids"].cpu().numpy()[ok], o["res"]["cut_id"][ok])
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("rows,V,bf16,mask,chunks", [
+    ([0, 1, 2, 3, 4, 5, 6, 7], 4097, False, False, 1), ([0, 8, 9, 10, 11, 12, 13], 4099, True, True, 1),
+    ([1, 9, 11, 13], 8192, True, False, 2), ([0, 3, 10], 16383, False, False, 3), ([2, 4, 8, 12], 12289, True, True, 3)])
+def test_short_rows_in_the_simulation(oracle, rows, V, bf16, mask, chunks):
+    """Rows that one workgroup's registers could hold, batches of every kind:
+    one chunk or a few."""
+    import sim as S
+
+    S.build()
+    x, p, u, h, hl, table = _topk_rows(oracle, V, 9 + V, bf16, mask)
+    x, p, u, h, hl = x[rows], p[rows], u[rows], h[rows], hl[rows]
+    o = oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=1025, want_post=True, nthreads=8)
+    for kept_cap in (1025, 0):  # with the kept lists and without them
+        r = S.run_sample(x, p, u, h, hl, mask_table=table, kept_cap=kept_cap, concurrent=True, repeat=2,
+                         env_extra={"TGS_KEY_SPINS": "100000"})
+        assert r["launches"] == [(len(rows) * chunks, 512)] * 2
+        if kept_cap:
+            H.compare(r, o, p, V, what="short rows")
+        else:
+            np.testing.assert_array_equal(r["ids"], o["ids"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,bf16,mask,hist", [
+    (4097, False, False, 64), (4104, True, True, 0), (7325, True, False, 64), (11008, False, True, 1000),
+    (16384, False, False, 64), (16385, True, True, 64), (32768, True, False, 0)])
+@pytest.mark.parametrize("copies", [1, 30])
+def test_short_rows(sampler, oracle, V, bf16, mask, hist, copies):
+    """Few rows over several chunks each, and more rows than CUs (one chunk up
+    to 16,384 ids)."""
+    x, p, u, h, hl, table = _topk_rows(oracle, V, V + 5, bf16, mask, hist)
+    rep = lambda t: None if t is None else np.concatenate([t] * copies)  # noqa: E731
+    x, p, u, h, hl = (rep(t) for t in (x, p, u, h, hl))
+    o = oracle.sample_batch(x, p, u, hist=h, hist_len=hl, mask_table=table, kept_cap=1025, want_post=True, nthreads=8)
+    H.log(f"case short rows V={V} bf16={bf16} mask={mask} B={len(p)}")
+    H.compare(H.run_gpu(sampler, x, p, u, h, hl, mask_table=table, kept_cap=1025), o, p, V, what="short rows")
+    import torch
+
+    import tinygpt_amd as tg
+
+    got = {"counts": torch.zeros(len(p), 2, dtype=torch.int32, device="cuda:0"),
+           "mass": torch.zeros(len(p), 2, dtype=torch.int64, device="cuda:0"),
+           "cut_ids": torch.zeros(len(p), dtype=torch.int32, device="cuda:0")}
+    ids = sampler.sample(H.to_dev(x), tg.params_to_device(p, "cuda:0"), H.to_dev(u), hist=H.to_dev(h),
+                         hist_len=H.to_dev(hl), vocab=V, debug=got)
+    np.testing.assert_array_equal(ids.cpu().numpy(), o["ids"])
+    ok = o["ids"] != -2
+    res = o["res"]
+    np.testing.assert_array_equal(got["counts"].cpu().numpy()[ok], np.stack([res["n_topk"], res["n_topp"]], 1)[ok])
+    np.testing.assert_array_equal(got["mass"].cpu().numpy().view(np.uint64)[ok],
+                                  np.stack([res["mass_k"], res["mass_p"]], 1)[ok])
+    np.testing.assert_array_equal(got["cut_ids"].cpu().numpy()[ok], res["cut_id"][ok])

@@ -144,10 +144,23 @@ int choose_split(int num_cu, int ws_rows, int B, int V) {
 // least what its registers need, chunks of at least 4096 ids (below that the
 // row's exchanges outweigh the work a further chunk takes over), in slabs the
 // workspace holds.
+constexpr int kSplitMin = 4096;  // least ids of a chunk
 int choose_split_topp(int num_cu, int B, int V) {
   const int smin = (V + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
-  const int S = std::min({tgs::TOPPS_MAX_SPLIT, num_cu / std::max(B, 1), V / 4096});
+  const int S = std::min({tgs::TOPPS_MAX_SPLIT, num_cu / std::max(B, 1), V / kSplitMin});
   return std::max(S, smin);
+}
+
+// Whether the split kernel takes a batch of every kind of row: rows beyond one
+// workgroup's registers always; shorter ones of more than kSplitMin ids
+// instead of the chunk, merge, full-path and top-p launches (41 mixed rows of
+// 11,008 fp32 ids 75 -> 33 us, 1000 of 16,000 135 -> 61, 223 of 7,325 bf16 with
+// k up to 1024 56 -> 30). Rows of two chunks only while the launch stays
+// within two workgroups per CU: 200 mixed rows of 32,000 139 -> 54, but 500
+// top-p rows of 20,000 without a hint take 50 there and 47 by the old launches.
+bool split_takes(int num_cu, int B, int V) {
+  if (V <= kSplitMin || V > tgs::topp_resident_ids()) return V > kSplitMin;
+  return V <= tgs::TOPPS_CHUNK || B <= num_cu;
 }
 
 // Static LDS of the fused kernel beyond its dynamic carve-up (wave lists,
@@ -210,9 +223,9 @@ int efail(std::string& err, int code, const std::string& msg) {
 // The rows without a top-k (all of a batch's, greedy rows too, with
 // a.topp_all): one workgroup per row where a row fits its registers, several
 // per row beyond.
-int topp_core(const SampleRes& res, std::string& err, tgs::SampleArgs a, tgs_dtype dt, hipStream_t stream) {
+int topp_core(const SampleRes& res, std::string& err, tgs::SampleArgs a, tgs_dtype dt, bool split, hipStream_t stream) {
   hipError_t e;
-  if (a.V > tgs::topp_resident_ids()) {
+  if (split) {
     const int S = choose_split_topp(res.num_cu, a.B, a.V);
     const int rows = (int)(res.ws_words / tgs::TOPPS_PAIR / (size_t)S);
     if (rows < 1) return efail(err, TGS_ETOOBIG, "workspace too small for top-p rows");
@@ -368,12 +381,11 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     // batch alone, greedy rows included
     a.full_rows = 1;
     a.topp_all = 1;
-    return topp_core(res, err, a, dt, stream);
+    return topp_core(res, err, a, dt, V > tgs::topp_resident_ids(), stream);
   }
   a.full_rows = (mk > tgs::KMAX || mk >= V) ? 1 : 0;
-  // rows beyond a workgroup's registers: the split kernel takes every kind
-  if (V > tgs::topp_resident_ids() && tgs::topp_lds_bytes(V, a.TS) + tgs::topps_static_lds() + 256 <= res.lds_limit)
-    return topp_core(res, err, a, dt, stream);
+  if (split_takes(res.num_cu, B, V) && tgs::topp_lds_bytes(V, a.TS) + tgs::topps_static_lds() + 256 <= res.lds_limit)
+    return topp_core(res, err, a, dt, true, stream);
   const int S = choose_split(res.num_cu, res.ws_rows, B, V);
   const int L = S > 1 ? ((V + S - 1) / S + 1023) / 1024 * 1024 : V;
   a.ws_stride = tgs::KMAX;
@@ -391,7 +403,7 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS (top-p rows)");
   hipError_t e = tgs::launch_sample(a, dt, lds, stream);
   if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
-  return a.full_rows ? topp_core(res, err, a, dt, stream) : TGS_OK;
+  return a.full_rows ? topp_core(res, err, a, dt, V > tgs::topp_resident_ids(), stream) : TGS_OK;
 }
 
 // ---------------------------------------------------------------- allocation-free sampling
@@ -542,7 +554,7 @@ int tgs_create(tgs_handle* out, int device, int max_batch, int max_vocab, int ma
   h->ws_rows = std::max(max_batch, 4 * h->num_cu);
   // (and room for the slabs of the split top-p kernel's chunks, at most 1024 at a time)
   size_t pairs = 0;
-  if (max_vocab > tgs::topp_resident_ids()) {
+  if (max_vocab > kSplitMin) {
     const int smin = (max_vocab + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
     pairs = std::max((size_t)std::min(h->num_cu, max_batch * tgs::TOPPS_MAX_SPLIT), (size_t)max_batch * smin);
     pairs = std::min(pairs, (size_t)1024);

@@ -1,7 +1,8 @@
 // tgs_topp_split.hip -- rows that sample with top-p over a vocabulary too
 // long for one workgroup's registers (tgs_topp.hip holds those), each row
 // over S workgroups of 512 threads in one launch; in a launch that serves
-// the whole batch, the greedy rows too.
+// the whole batch, the greedy rows too.  Batches of every kind of row come
+// here from 4,097 ids on; a row of one chunk skips the exchanges.
 //
 // What bounds it: one workgroup streams a row at one CU's rate and evaluates
 // every id's exact mass (about 40 VALU operations) on one CU, three passes
@@ -220,6 +221,29 @@ __device__ __forceinline__ void finish_topk(const SampleArgs& a, const Row& r, u
   }
 }
 
+// A y below the k-th largest (k <= the allowed ids, or -inf) of a row held by
+// one workgroup, from counts per bucket of 1/32 below its maximum: for k
+// above the thread count, which no thread maxima bound.  RN(m - y) <
+// (q + 1) / 32 gives y > m - (q + 2) / 32, and so y >= its rounding.  CI and
+// MI are zero before; ends with a barrier.
+template <typename Tin>
+__device__ __forceinline__ float counted_floor(const RowView<Tin, true, SBT>& rv, u64 mc, unsigned k, Tail& tl,
+                                               SplitShared& sh) {
+  const u64 Mc = block_reduce_max<SBT>(mc, sh.ts.red64);
+  const float m = Mc ? comp_y(Mc) : 0.0f;
+#pragma unroll
+  for (int q = 0; q < RES_EPT; q++) {
+    const float y = rv.y[q];
+    const float f = y == m ? 0.0f : (m - y) * 32.0f;
+    if (y > -__builtin_inff()) atomicAdd(&tl.CI[f < (float)NB ? (int)f : NB], 1u);
+  }
+  __syncthreads();
+  bucket::prefix<SBT>(tl.CI, tl.MI, sh.ts.red32, sh.ts.red64);
+  if (tl.CI[NB - 1] < k) return -__builtin_inff();
+  const int q = bucket::find_count<SBT>(tl.CI, k, &sh.ts.sel[0]);
+  return m - (float)(q + 2) * 0.03125f;
+}
+
 // The decision word: the epoch's low 24 bits over the list buckets in 40
 // (bit 0: they are to be gathered; a run of 512 buckets or more for list B is
 // settled by the owner alone).  Every call of a row writes it, so a stale one
@@ -306,18 +330,27 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
   }
 
+  // a top-k past one wave's lists (of one chunk), or past what S short lists
+  // hold, whose kept list nobody asked for goes through the histograms like a
+  // larger one: the list's cut, mass and draw each select by digits, and lists
+  // beyond CAPL select the set first (223 rows of 7,325 bf16 ids, k up to 1024:
+  // 58 -> 30 us; 200 mixed rows of 32,000 109 -> 54).  Over more chunks the
+  // list has one meeting against three (41 mixed rows of 11,008: 29 by lists
+  // alone, 33 with this rule)
+  const bool hist_k = r.k > (a.S == 1 ? 64 : 256 * a.S) && !a.dbg.kept_ids && !a.dbg.kept_probs;
   u64 mc = thread_best<Tin, SBT>(rv);
   u64* slab = a.ws + ((long long)lb * a.S + c) * TOPPS_PAIR;
   const u64* slabs = a.ws + (long long)lb * a.S * TOPPS_PAIR;
   if (threadIdx.x == 0) sh.ts.ng = 0;
 
-  if (r.mode == 1) {
+  if (r.mode == 1 && !hist_k) {
     // ---- a top-k of at most KMAX: the chunk's ids that reach a floor under
     // the row's k-th largest y, and no more meetings.  Floors from the thread
     // maxima (bound_key): the chunk's own k-th largest (k <= SBT), or, when S
     // lists of that many would be too long (meet), the lowest over the chunks
     // of each one's ceil(k / S)-th largest, or the highest of their k-th.
-    const bool meet = 2 * a.S * r.k > CAPL;
+    const bool counted = a.S == 1 && 4 * r.k > 3 * SBT;
+    const bool meet = a.S > 1 && (2 * a.S * r.k > CAPL || 2 * r.k > SBT);
     const int k2 = (r.k + a.S - 1) / a.S;
     const uint32_t srt = wave_sort_desc((uint32_t)(mc >> 32));
 #pragma unroll
@@ -343,7 +376,8 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       __syncthreads();
       kb = sh.floor > kb ? sh.floor : kb;
     }
-    const float yb = kb ? tg_unkey(kb) : -__builtin_inff();
+    float yb = kb ? tg_unkey(kb) : -__builtin_inff();
+    if (counted) yb = counted_floor<Tin>(rv, mc, (unsigned)r.k, tl, sh);
     gather_floor(rv, yb, sh.ts, [&](unsigned o, u64 x) {
       if (o < (unsigned)TOPPS_PAIR) st(slab + o, x);
     });
@@ -444,13 +478,16 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   }
   if (w == 0) {
     mc = wave_max(lane < SBT / 64 ? sh.ts.red64[lane] : 0ull);
-    if (lane == 0) st(maxima + c, max_entry(mc, ep));
-    u64 e;
-    const bool ok = poll_words(maxima, a.S, ep, a.key_spins, &e);
-    // (entries of the call order as their composites)
-    const u64 x = wave_max(ok ? e : 0ull);
+    bool ok = true;
+    if (a.S > 1) {
+      if (lane == 0) st(maxima + c, max_entry(mc, ep));
+      u64 e;
+      ok = poll_words(maxima, a.S, ep, a.key_spins, &e);
+      // (entries of the call order as their composites)
+      mc = max_comp(wave_max(ok ? e : 0ull));
+    }
     if (lane == 0) {
-      sh.rowmax = max_comp(x);
+      sh.rowmax = mc;
       sh.flag = ok;
     }
   }
@@ -472,18 +509,20 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   // ---- 2. the chunk's histogram, its slab, and the arrival
   if (sampling) {
     histogram(rv, tl);
-    __syncthreads();
-    unsigned* sc = (unsigned*)(slab + NB);
-    for (int i = threadIdx.x; i < NB; i += SBT) {
-      st(slab + i, tl.MI[i]);
-      st(sc + i, tl.CI[i]);
+    if (a.S > 1) {
+      __syncthreads();
+      unsigned* sc = (unsigned*)(slab + NB);
+      for (int i = threadIdx.x; i < NB; i += SBT) {
+        st(slab + i, tl.MI[i]);
+        st(sc + i, tl.CI[i]);
+      }
+      if (threadIdx.x == 0) st(sc + NB, tl.CI[NB]);
+      wait_stores();
     }
-    if (threadIdx.x == 0) st(sc + NB, tl.CI[NB]);
-    wait_stores();
   }
   __syncthreads();
   if (threadIdx.x == 0)
-    sh.arrived = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sh.arrived = a.S > 1 ? __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
   __syncthreads();
   const bool owner = sh.arrived == (unsigned)(a.S - 1);
   if (!owner && !sampling) return;
@@ -530,7 +569,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     write_greedy<SBT>(a, r, Mc);
     if (threadIdx.x == 0) st(decision, (u64)0);
   } else {
-    {
+    if (a.S > 1) {
       // thread t sums buckets t and t + 512, eight slabs' words in flight
       u64 ms[2] = {0ull, 0ull};
       unsigned cs[2] = {0u, 0u};
@@ -562,7 +601,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
         tl.CI[threadIdx.x + h * SBT] = cs[h];
       }
     }
-    if (w == 0) {
+    if (a.S > 1 && w == 0) {
       unsigned x = lane < a.S ? ld((const unsigned*)(slabs + (long long)lane * TOPPS_PAIR + NB) + NB) : 0u;
       x = wave_sum(x);
       if (lane == 0) tl.CI[NB] = x;
@@ -572,11 +611,12 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     const unsigned nall = tl.CI[NB];
     const unsigned kk = has_k && (unsigned)r.k < nall ? (unsigned)r.k : nall;
     Plan pl;
-    bool lists = true;
-    if (kk == nall) plan_row<SBT>(pl, r, tl, Mc, nall, sh.ts);
-    else if (kk <= tl.CI[NB - 1]) plan_topk<SBT>(pl, r, tl, Mc, kk, sh.ts);
-    else lists = false;  // the top-k set reaches the mass-0 bucket
-    lists = lists && packs(pl);
+    // a top-k set that reaches the mass-0 bucket carries the whole row's mass:
+    // only its last element (a cut with top-p off) is still its own
+    const bool whole = kk == nall || kk > tl.CI[NB - 1];
+    if (whole) plan_row<SBT>(pl, r, tl, Mc, kk, sh.ts);
+    else plan_topk<SBT>(pl, r, tl, Mc, kk, sh.ts);
+    const bool lists = packs(pl);
     if (threadIdx.x == 0) st(decision, (u64)(ep & 0xFFFFFFu) << 40 | (lists ? pack_plan(pl) : 0ull));
     SV sv(a, r, hash, hbits, rowp);
     u64 pick;
@@ -645,11 +685,22 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       __syncthreads();
       pick = pick_gathered<SBT>(pl, r.top_p, tl, sh.ts, sh.bs);
     } else {
-      if (kk < nall) {
+      if (!whole) {
         pick = pick_streamed<SBT>(pl, kk, r, sv, Mc, tl, sh.ts, sh.bs);
       } else {
         pick = pick_resolved<SBT>(pl, sv, tl, sh.ts, sh.bs);
       }
+    }
+    if (kk < nall && whole && pl.cut_last && a.dbg.cut_ids) {
+      const u64 T = block_select_kth<u64, 64, SBT>(
+          [&](auto f) { sv.each([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, kk, sh.bs);
+      u64 x = 0ull;
+      sv.each([&](int id, float y) {
+        const u64 v = comp_key(tg_key(y), id);
+        if (v >= T) x = ~v > x ? ~v : x;
+      });
+      pl.cutc = ~block_max<u64, SBT>(x, sh.ts.red64);
+      pl.cut_last = false;
     }
     write_row<SBT>(a, b, pl, pick, sv, sh.ts);
   }
