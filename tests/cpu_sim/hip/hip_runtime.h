@@ -12,7 +12,8 @@
 // object gets a copy per block instead.  With TGS_SIM_CONCURRENT set, every
 // block of a launch runs at once (for kernels whose blocks wait on each
 // other; only kernels with no plain __shared__ variables may run so).
-// Device memory is host memory.
+// Device memory is host memory.  TGS_SIM_STAGGER makes the waves of a block run
+// apart between barriers.
 #pragma once
 
 #include <atomic>
@@ -242,7 +243,21 @@ inline void launch(void (*k)(Args...), dim3 grid, dim3 block, size_t shmem, Args
 
 #define hipLaunchKernelGGL(k, g, b, sh, st, ...) hipcpu::launch(k, dim3(g), dim3(b), (size_t)(sh), __VA_ARGS__)
 
-inline void __syncthreads() { hipcpu::block_ctx()->bar->arrive_and_wait(); }
+// TGS_SIM_STAGGER=us: after every workgroup barrier the waves go on one after
+// another, that long apart (another one first at each barrier), so that a word
+// that one wave reads there and another writes is written first.
+inline void hipcpu_stagger() {
+  static const int us = std::getenv("TGS_SIM_STAGGER") ? std::atoi(std::getenv("TGS_SIM_STAGGER")) : 0;
+  static thread_local unsigned turn = 0;
+  if (us <= 0) return;
+  const unsigned nw = (hipcpu::g_block_dim.x + 63) / 64;
+  const unsigned place = (hipcpu::t_thread.x / 64 + turn++) % nw;
+  if (place) usleep((unsigned)us * place);
+}
+inline void __syncthreads() {
+  hipcpu::block_ctx()->bar->arrive_and_wait();
+  hipcpu_stagger();
+}
 inline int __syncthreads_or(int pred) {
   static std::atomic<int> acc{0};
   __syncthreads();

@@ -66,6 +66,23 @@ def test_fast_kernel_with_hint(sim, oracle):
     _check(sim, oracle, x, params, u, hist, hist_len, hint=tg.batch_hint(params, 300))
 
 
+def test_chunk_kernel_waves_apart(sim, oracle):
+    """Top-k rows whose first tile leaves between CAPB / 2 and CAPB candidates
+    (k = 768: the 256th largest of the threads' third maxima), with the waves
+    of a workgroup running apart after every barrier: all of them take the
+    same branch on the candidate count, whatever a faster one has appended."""
+    g = np.random.default_rng(0)
+    B, V = 4, 3000
+    x = (g.standard_normal((B, V)) * 3.0).astype(np.float32)
+    params = oracle.make_params(B, temperature=0.9, top_k=0, top_p=0.95)
+    params["top_k"] = [768, 760, 764, 256]
+    u = (g.integers(0, 1 << 24, B) / (1 << 24)).astype(np.float32)
+    r = sim.run_sample(x, params, u, kept_cap=1025, env_extra={"TGS_SIM_STAGGER": "10000"})
+    assert r["launches"][0] == (B, 256)  # the chunk kernel
+    o = oracle.sample_batch(x, params, u, kept_cap=1025, want_post=True)
+    H.compare(r, o, params, V, what="sim")
+
+
 def test_split_rows_and_merge(sim, oracle):
     x, params, u, hist, hist_len = _batch(13, 4, 5000, oracle)
     _check(sim, oracle, x, params, u, hist, hist_len, split=3)

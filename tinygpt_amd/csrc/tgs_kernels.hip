@@ -440,7 +440,7 @@ __device__ __forceinline__ void topk_chunk(const SampleArgs& a, const Row& r, co
   const Tin* rowp = (const Tin*)a.logits + (long long)r.b * a.row_stride;
   float* post = a.dbg.post_logits ? a.dbg.post_logits + (long long)r.b * a.V : nullptr;
   const int k = r.k;
-  if (threadIdx.x == 0) s.nbuf = 0;
+  if (threadIdx.x == 0) s.nbuf = 0;  // (read past first_threshold's barriers)
   u64 thr = 0;  // candidates: composite >= thr and key != 0
   uint32_t key[TL::EPT];
   bool first = true;
@@ -452,8 +452,11 @@ __device__ __forceinline__ void topk_chunk(const SampleArgs& a, const Row& r, co
       first = false;
     }
     uint32_t cm = cand_mask<TL::EPT, TL::EPV>(key, t0, thr);
-    const unsigned total = block_sum((unsigned)__popc(cm), s.red32);
+    // the count is read ahead of the sum's barriers: no wave appends before
+    // every wave has read it (read behind them, a wave that came late counted
+    // what a faster one had appended, and took the branch below alone)
     const unsigned nbuf = s.nbuf;
+    const unsigned total = block_sum((unsigned)__popc(cm), s.red32);
     if (nbuf + total > (unsigned)CAPB) {
       // shrink: exact k-th composite over the buffer and this tile's candidates
       const uint32_t cm_old = cm;
