@@ -26,6 +26,7 @@
 #include <memory>
 #include <thread>
 #include <type_traits>
+#include <utility>
 #include <vector>
 
 #include <linux/futex.h>
@@ -405,9 +406,16 @@ inline int& hipcpu_last_error() {
 }
 inline hipError_t hipGetLastError() { int e = hipcpu_last_error(); hipcpu_last_error() = 0; return e; }
 inline const char* hipGetErrorString(hipError_t e) { return e ? "hipcpu error" : "no error"; }
+// Every allocation so far and its size (tests that set state which a handle
+// carries from call to call find it here).
+inline std::vector<std::pair<void*, size_t>>& hipcpu_allocations() {
+  static std::vector<std::pair<void*, size_t>> v;
+  return v;
+}
 template <typename T>
 inline hipError_t hipMalloc(T** p, size_t n) {
   *p = (T*)std::malloc(n ? n : 1);
+  hipcpu_allocations().emplace_back((void*)*p, n);
   return *p ? hipSuccess : hipErrorOutOfMemory;
 }
 inline hipError_t hipFree(void* p) { std::free(p); return hipSuccess; }

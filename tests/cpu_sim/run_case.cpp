@@ -2,6 +2,8 @@
 // CPU simulation of the kernels (TEST INFRASTRUCTURE ONLY).
 //   run_case sample <dir>   reads <dir>/meta.txt and the raw input arrays,
 //                           writes the outputs next to them.
+//   run_case sequence <dir> calls on one handle, one after another (the state
+//                           that a handle carries from call to call).
 #include <cstdint>
 #include <cstdio>
 #include <algorithm>
@@ -13,6 +15,7 @@
 #include <unistd.h>
 
 #include "../../include/tgs_sampler.h"
+#include "tgs_kernels.h"
 
 static std::vector<char> slurp(const std::string& path) {
   std::vector<char> v;
@@ -129,6 +132,53 @@ int main(int argc, char** argv) {
     dump(dir + "/out_mass.bin", mass.data(), mass.size() * 8);
     dump(dir + "/out_cut.bin", cut.data(), cut.size() * 4);
     if (post) dump(dir + "/out_post.bin", postv.data(), postv.size() * 4);
+    tgs_destroy(h);
+    return 0;
+  }
+  if (mode == "sequence") {
+    // meta.txt: max B, max V, max history, mask states, calls; then per call
+    // B, V, hint (-1: none), its min_top_k, and the epoch word to set in every
+    // row's exchange line of the split kernel before it (-1: as it is), which
+    // stands for that many calls before.  Inputs of call i: <name>.<i>.bin
+    // (fp32 logits [B][V], history [B][max history] when there is one).
+    int mb, mv, mh, n_states, calls;
+    if (std::fscanf(m, "%d %d %d %d %d", &mb, &mv, &mh, &n_states, &calls) != 5) return 4;
+    tgs_handle h;
+    int rc = tgs_create(&h, 0, mb, mv, mh);
+    if (rc) { std::printf("create %d\n", rc); return 5; }
+    // the handle's zeroed allocation: fused-kernel lists, keys, the split
+    // kernel's lines, the fused kernel's lines
+    const size_t lists = (size_t)mb * tgs::K64_MAX_SPLIT * 64, keys = (size_t)mb * tgs::K64_KEYS;
+    const size_t need = 8 * (lists + keys + (size_t)mb * tgs::TOPPS_LINE) + 4 * (size_t)mb * tgs::K64_CNT_STRIDE;
+    unsigned long long* lines = nullptr;
+    for (const auto& e : hipcpu_allocations())
+      if (e.second == need) lines = (unsigned long long*)e.first + lists + keys;
+    if (!lines) { std::printf("the zeroed allocation is laid out in another way\n"); return 10; }
+    auto mask = slurp(dir + "/mask.bin");
+    if (n_states > 0) {
+      rc = tgs_mask_table_set(h, (const uint32_t*)mask.data(), n_states, mv);
+      if (rc) { std::printf("mask %d\n", rc); return 6; }
+    }
+    for (int i = 0; i < calls; i++) {
+      int B, V, hint, hint_min;
+      long long epoch;
+      if (std::fscanf(m, "%d %d %d %d %lld", &B, &V, &hint, &hint_min, &epoch) != 5) return 4;
+      const std::string at = "." + std::to_string(i) + ".bin";
+      auto logits = slurp(dir + "/logits" + at), params = slurp(dir + "/params" + at), u = slurp(dir + "/u" + at);
+      auto hist = slurp(dir + "/hist" + at);
+      if (epoch >= 0)
+        for (int b = 0; b < mb; b++) ((unsigned*)(lines + (size_t)b * tgs::TOPPS_LINE))[1] = (unsigned)epoch;
+      tgs_batch_hint hb = {hint, hint_min};
+      std::vector<int32_t> out(B);
+      std::printf("call %d\n", i);
+      std::fflush(stdout);
+      rc = tgs_sample(h, logits.data(), TGS_F32, B, V, V, mh ? (const int32_t*)hist.data() : nullptr, nullptr, mh,
+                      (const tgs_row_params*)params.data(), (const float*)u.data(), out.data(),
+                      hint >= 0 ? &hb : nullptr, nullptr, nullptr);
+      if (rc) { std::printf("sample %d %s\n", rc, tgs_last_error(h)); return 7; }
+      dump(dir + "/ids" + at, out.data(), out.size() * 4);
+    }
+    std::fclose(m);
     tgs_destroy(h);
     return 0;
   }

@@ -101,6 +101,42 @@ def run_sample(logits, params, u, hist=None, hist_len=None, mask_table=None, V=N
         return r
 
 
+def run_sequence(calls, mask_table=None, alarm=60, env_extra=None):
+    """Calls on one handle, every workgroup of a launch running at once.
+    calls: dicts of x (float32 [B, V]), p, u, hist (None, or int32 [B, H] with
+    the same H in every call), hint (None or a batch_hint) and epoch (None, or
+    the epoch word set before the call in every row's exchange line of the
+    split kernel).  A run of more than `alarm` seconds is stopped and fails.
+    Returns the calls' ids."""
+    H = max(0 if c.get("hist") is None else c["hist"].shape[1] for c in calls)
+    with tempfile.TemporaryDirectory(dir=os.environ.get("TMPDIR", "/tmp")) as d:
+        lines = []
+        for i, c in enumerate(calls):
+            B, V = c["x"].shape
+            put = lambda name, a, dt: np.ascontiguousarray(a, dt).tofile(os.path.join(d, f"{name}.{i}.bin"))  # noqa: E731
+            put("logits", c["x"], np.float32)
+            put("u", c["u"], np.float32)
+            put("params", c["p"], c["p"].dtype)
+            if H:
+                put("hist", c["hist"], np.int32)
+            hint, epoch = c.get("hint"), c.get("epoch")
+            lines.append(f"{B} {V} {-1 if hint is None else int(hint)} {int(getattr(hint, 'min_top_k', 0))} "
+                         f"{-1 if epoch is None else epoch}")
+        n_states = 0
+        if mask_table is not None:
+            n_states = mask_table.shape[0]
+            np.ascontiguousarray(mask_table, np.uint32).tofile(os.path.join(d, "mask.bin"))
+        mb, mv = max(c["x"].shape[0] for c in calls), max(c["x"].shape[1] for c in calls)
+        with open(os.path.join(d, "meta.txt"), "w") as f:
+            f.write(f"{mb} {mv} {H} {n_states} {len(calls)}\n" + "\n".join(lines) + "\n")
+        env = {**os.environ, "TGS_SIM_CONCURRENT": "1", "TGS_KEY_SPINS": "100000", "TGS_SIM_ALARM": str(alarm),
+               **(env_extra or {}), **_san_env()}
+        r = subprocess.run([BIN, "sequence", d], capture_output=True, text=True, env=env, timeout=alarm + 60)
+        if r.returncode != 0:
+            raise RuntimeError(f"run_case exit {r.returncode}\n{r.stdout[-4000:]}\n{r.stderr[-12000:]}")
+        return [np.fromfile(os.path.join(d, f"ids.{i}.bin"), np.int32) for i in range(len(calls))]
+
+
 def run_maskbuild(byte_class, trans, complete, tok_off, tok_bytes, states, rows, n_rows, eos=-1, timeout=600):
     """tgs_mask_rows_from_dfa through the simulation (trans [n_dfa, n_cls]),
     read back as the post_logits of greedy rows over zero logits: float32

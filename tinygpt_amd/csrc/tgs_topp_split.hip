@@ -85,6 +85,9 @@ __device__ __forceinline__ void st(T* p, T v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The decision word (see pack_plan) without lists to gather.
+__device__ __forceinline__ u64 decision_tag(uint32_t ep) { return (u64)(ep & 0xFFFFFFu) << 40; }
+
 // A chunk's largest composite with the epoch's low bits between key and id
 // (never 0; entries of one call order as their composites; key 0: nothing
 // allowed).
@@ -102,10 +105,19 @@ __device__ __forceinline__ u64 max_comp(u64 e) {
 }
 
 // Ready for the next call: counter zero, maxima cleared, epoch advanced
-// (every workgroup of the row has arrived, so nothing polls the maxima).
-__device__ __forceinline__ void reset_line(const SampleArgs& a, unsigned* cnt, u64* maxima, uint32_t ep) {
-  if (threadIdx.x < (unsigned)a.S) st(maxima + threadIdx.x, (u64)0);
+// (every workgroup of the row has arrived, so nothing polls the maxima), and
+// a decision of this epoch with nothing to gather.  Every ending of a row
+// leaves one, so the word that a call finds is always its predecessor's, one
+// epoch back: a word left from before (or never written, which reads as epoch
+// 0) would pass for current once the 24 bits of the tag come round, after
+// 2^24 calls whose rows had nothing to decide.  A workgroup that still polls
+// finds what the owner published: one whose lists the owner waits for has
+// left by now, and without lists the word is the same.
+__device__ __forceinline__ void reset_line(const SampleArgs& a, u64* line, uint32_t ep) {
+  unsigned* cnt = (unsigned*)line;
+  if (threadIdx.x < (unsigned)a.S) st(line + 2 + threadIdx.x, (u64)0);
   if (threadIdx.x == 0) {
+    st(line + 1, decision_tag(ep));
     st(cnt, 0u);
     st(cnt + 1, ep == 0xFFFFFFFFu ? 0u : ep);
   }
@@ -246,8 +258,8 @@ __device__ __forceinline__ float counted_floor(const RowView<Tin, true, SBT>& rv
 
 // The decision word: the epoch's low 24 bits over the list buckets in 40
 // (bit 0: they are to be gathered; a run of 512 buckets or more for list B is
-// settled by the owner alone).  Every call of a row writes it, so a stale one
-// is the previous call's.
+// settled by the owner alone).  Every ending of a row leaves the word with
+// its epoch (reset_line), so a stale one is the previous call's.
 __device__ __forceinline__ bool packs(const Plan& pl) { return pl.one && pl.b1 - pl.b0 < 511; }
 __device__ __forceinline__ u64 pack_plan(const Plan& pl) {
   return 1ull | (u64)pl.a0 << 1 | (u64)pl.a1 << 11 | (u64)pl.b0 << 21 | (u64)(pl.b1 - pl.b0 + 1) << 31;
@@ -447,7 +459,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       __syncthreads();
       finish_topk(a, r, tl.L, n, tl, sh);
     }
-    reset_line(a, cnt, maxima, ep);
+    reset_line(a, line, ep);
     return;
   }
 
@@ -473,7 +485,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
     __syncthreads();
     write_greedy<SBT>(a, r, sh.rowmax);
-    reset_line(a, cnt, maxima, ep);
+    reset_line(a, line, ep);
     return;
   }
   if (w == 0) {
@@ -567,7 +579,6 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   // ---- the owner: the row's histogram, the cut and the draw
   if (!sampling) {
     write_greedy<SBT>(a, r, Mc);
-    if (threadIdx.x == 0) st(decision, (u64)0);
   } else {
     if (a.S > 1) {
       // thread t sums buckets t and t + 512, eight slabs' words in flight
@@ -617,7 +628,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     if (whole) plan_row<SBT>(pl, r, tl, Mc, kk, sh.ts);
     else plan_topk<SBT>(pl, r, tl, Mc, kk, sh.ts);
     const bool lists = packs(pl);
-    if (threadIdx.x == 0) st(decision, (u64)(ep & 0xFFFFFFu) << 40 | (lists ? pack_plan(pl) : 0ull));
+    if (threadIdx.x == 0) st(decision, decision_tag(ep) | (lists ? pack_plan(pl) : 0ull));
     SV sv(a, r, hash, hbits, rowp);
     u64 pick;
     if (lists) {
@@ -704,7 +715,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
     write_row<SBT>(a, b, pl, pick, sv, sh.ts);
   }
-  reset_line(a, cnt, maxima, ep);
+  reset_line(a, line, ep);
 }
 
 }  // namespace topp
