@@ -82,3 +82,11 @@ def test_kinds_and_lengths_alternate(oracle, word):
     calls = [_call(oracle, k, V, seed=20 + i) for i, (k, V) in enumerate(zip(kinds, lengths))]
     calls[0]["epoch"] = word
     _run(oracle, calls)
+
+
+@sim
+def test_done_words_come_round(oracle):
+    """Lists published 2^32 - 1 calls ago, all between without any: they are
+    not taken for the current call's."""
+    _run(oracle, [_call(oracle, "topp", seed=40), _call(oracle, "greedy", seed=41, epoch=(1 << 32) - 2),
+                  _call(oracle, "topp", seed=42)])

@@ -34,8 +34,9 @@
 // The exchange uses agent-scope loads and stores throughout (they pass the
 // per-XCD L2s, which are not coherent with each other) and plain waits for
 // the issuing wave's stores; no fence is issued (an agent-scope fence writes
-// back or invalidates a whole L2).  Words carry the call's epoch, so nothing
-// needs clearing between calls except the maxima, whose tag is short.
+// back or invalidates a whole L2).  Words carry the call's epoch, and the
+// row's owner leaves none behind that a later call could take for its own
+// (reset_line).
 //
 // Measured against one workgroup per row streaming it three times (per call):
 // 1 row of 151,936 bf16 ids with penalties 137 -> 30 us, 32 rows of 128,256
@@ -104,18 +105,24 @@ __device__ __forceinline__ u64 max_comp(u64 e) {
   return (e >> 32) ? comp_key((uint32_t)(e >> 32), (int)(SIDM - (uint32_t)(e & SIDM))) : 0ull;
 }
 
-// Ready for the next call: counter zero, maxima cleared, epoch advanced
-// (every workgroup of the row has arrived, so nothing polls the maxima), and
+// Ready for the next call: counter zero, maxima and done words cleared, epoch
+// advanced (every workgroup of the row has arrived, so nothing polls the maxima), and
 // a decision of this epoch with nothing to gather.  Every ending of a row
 // leaves one, so the word that a call finds is always its predecessor's, one
 // epoch back: a word left from before (or never written, which reads as epoch
 // 0) would pass for current once the 24 bits of the tag come round, after
 // 2^24 calls whose rows had nothing to decide.  A workgroup that still polls
 // finds what the owner published: one whose lists the owner waits for has
-// left by now, and without lists the word is the same.
+// left by now, and without lists the word is the same.  The done words are
+// cleared for the same reason (the epoch itself comes round after 2^32
+// calls); only one that says its workgroup left without lists can still be on
+// its way, and the owner reads that chunk itself, which is right at any time.
 __device__ __forceinline__ void reset_line(const SampleArgs& a, u64* line, uint32_t ep) {
   unsigned* cnt = (unsigned*)line;
-  if (threadIdx.x < (unsigned)a.S) st(line + 2 + threadIdx.x, (u64)0);
+  if (threadIdx.x < (unsigned)a.S) {
+    st(line + 2 + threadIdx.x, (u64)0);
+    st(line + 2 + TOPPS_MAX_SPLIT + threadIdx.x, (u64)0);
+  }
   if (threadIdx.x == 0) {
     st(line + 1, decision_tag(ep));
     st(cnt, 0u);
