@@ -95,7 +95,7 @@ def test_topk_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("rows,V,bf16,mask,concurrent", [
     ([0, 1], 32769, False, False, True), ([2, 3], 33001, True, True, True), ([4, 5], 36864, False, True, True),
-    ([6, 7], 32800, True, False, True), ([0, 1, 2, 4], 33003, True, False, False), ([3, 5], 33002, False, True, False)])
+    ([6, 7], 32800, True, False, True), ([6, 5], 32800, True, False, False), ([0, 1, 2, 4], 33003, True, False, False), ([3, 5], 33002, False, True, False)])
 def test_split_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
     import sim as S
 

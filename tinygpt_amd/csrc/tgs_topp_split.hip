@@ -540,8 +540,12 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
   }
   __syncthreads();
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
+    // (its maximum too: a row with nothing allowed has stored only that, and
+    // the owner clears it once all have arrived)
+    wait_stores();
     sh.arrived = a.S > 1 ? __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+  }
   __syncthreads();
   const bool owner = sh.arrived == (unsigned)(a.S - 1);
   if (!owner && !sampling) return;
