@@ -95,7 +95,8 @@ def test_topk_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("rows,V,bf16,mask,concurrent", [
     ([0, 1], 32769, False, False, True), ([2, 3], 33001, True, True, True), ([4, 5], 36864, False, True, True),
-    ([6, 7], 32800, True, False, True), ([6, 5], 32800, True, False, False), ([0, 1, 2, 4], 33003, True, False, False), ([3, 5], 33002, False, True, False)])
+    ([6, 7], 32800, True, False, True), ([6, 5], 32800, True, False, False),
+    ([0, 1, 2, 4], 33003, True, False, False), ([3, 5], 33002, False, True, False)])
 def test_split_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
     import sim as S
 
@@ -109,6 +110,27 @@ def test_split_rows_in_the_simulation(oracle, rows, V, bf16, mask, concurrent):
                      repeat=2 if concurrent else 1, env_extra={"TGS_KEY_SPINS": "100000"} if concurrent else None)
     assert all(blk == 512 and grid > len(rows) for grid, blk in r["launches"])
     H.compare(r, _oracle(oracle, x, p, u, h, hl, table), p, V, what="split top-p")
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_slabs_of_the_static_workspace(oracle):
+    """A batch of 276 chunks takes one launch on the allocation-free entry
+    point's workspace too (all but one of its rows greedy)."""
+    import sim as S
+
+    import tinygpt_amd as tg
+
+    S.build()
+    B, V = 92, 32769
+    g = np.random.default_rng(92)
+    x = np.tile((g.standard_normal((1, V)) * 3.0).astype(np.float32), (B, 1))
+    x[np.arange(B), g.integers(0, V, B)] = 20.0
+    p = oracle.make_params(B, temperature=0.0, top_p=0.9)
+    p["temperature"][50] = 0.8
+    u = np.full(B, 0.75, np.float32)
+    r = S.run_sample(x, p, u, hint=tg.batch_hint(p, V), post=False, kept_cap=8, noalloc=True)
+    assert [n for n in r["launches"] if n[1] == 512] == [(3 * B, 512)]
+    np.testing.assert_array_equal(r["ids"], oracle.sample_batch(x, p, u, nthreads=8)["ids"])
 
 
 @pytest.mark.gpu

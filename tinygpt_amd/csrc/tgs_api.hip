@@ -145,6 +145,12 @@ int choose_split(int num_cu, int ws_rows, int B, int V) {
 // row's exchanges outweigh the work a further chunk takes over), in slabs the
 // workspace holds.
 constexpr int kSplitMin = 4096;  // least ids of a chunk
+// Slabs of a handle at most (15 KB each).  Each launch ends with the rows that
+// take longest alone on the chip: with 1024 slabs, 512 top-p rows of 151,936
+// bf16 ids took 360 us in five launches, with 4096 in two 284 (one workgroup
+// per row 310), 1024 of 33,000 205 and 150 (166).  The allocation-free entry
+// point holds kNaSlabs: with 272, 256 rows of 128,256 fp32 took 239 (166).
+constexpr int kSplitSlabs = 4096;
 int choose_split_topp(int num_cu, int B, int V) {
   const int smin = (V + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
   const int S = std::min({tgs::TOPPS_MAX_SPLIT, num_cu / std::max(B, 1), V / kSplitMin});
@@ -413,7 +419,7 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
 // the process ends) instead of a handle's allocations:
 //   [k64 chunk lists: kNaRows * kMaxSplit * 64 u64, entries 0 between calls]
 //   [k64 bound-exchange keys: kNaRows * K64_KEYS u64]
-//   [general-path chunk lists: kNaWsRows * KMAX u64]
+//   [general-path chunk lists, kNaWsRows * KMAX u64, or split-kernel slabs, kNaSlabs * TOPPS_PAIR u64]
 //   [split top-p exchange lines: kNaRows * TOPPS_LINE u64]
 //   [k64 exchange lines: kNaRows * K64_CNT_STRIDE u32, counters zero between calls]
 //   [general-path list counts: kNaWsRows * (KMAX / 64) i32]
@@ -424,10 +430,11 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
 // device comes from hipGetSymbolAddress.
 constexpr int kNaRows = 256;    // rows per call
 constexpr int kNaWsRows = 512;  // general-path (row, chunk) lists
+constexpr int kNaSlabs = 1024;  // split kernel (row, chunk) slabs, in the same words
 constexpr int kNaHist = tgs::K64_MAX_HIST;
 constexpr size_t kNaListWords = (size_t)kNaRows * kMaxSplitK64 * 64;
 constexpr size_t kNaKeyWords = (size_t)kNaRows * tgs::K64_KEYS;
-constexpr size_t kNaWsWords = (size_t)kNaWsRows * tgs::KMAX;
+constexpr size_t kNaWsWords = std::max((size_t)kNaWsRows * tgs::KMAX, (size_t)kNaSlabs * tgs::TOPPS_PAIR);
 constexpr size_t kNaTpWords = (size_t)kNaRows * tgs::TOPPS_LINE;
 constexpr size_t kNaCntU32 = (size_t)kNaRows * tgs::K64_CNT_STRIDE;
 constexpr size_t kNaWsCntI32 = (size_t)kNaWsRows * (tgs::KMAX / 64);
@@ -552,12 +559,13 @@ int tgs_create(tgs_handle* out, int device, int max_batch, int max_vocab, int ma
   if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device) == hipSuccess && v > 0)
     h->lds_limit = (size_t)v;
   h->ws_rows = std::max(max_batch, 4 * h->num_cu);
-  // (and room for the slabs of the split top-p kernel's chunks, at most 1024 at a time)
+  // (and room for the slabs of the split kernel's chunks; a batch of more
+  // chunks than kSplitSlabs takes several launches)
   size_t pairs = 0;
   if (max_vocab > kSplitMin) {
     const int smin = (max_vocab + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
     pairs = std::max((size_t)std::min(h->num_cu, max_batch * tgs::TOPPS_MAX_SPLIT), (size_t)max_batch * smin);
-    pairs = std::min(pairs, (size_t)1024);
+    pairs = std::min(pairs, (size_t)kSplitSlabs);
   }
   h->ws_words = std::max((size_t)h->ws_rows * tgs::KMAX, pairs * tgs::TOPPS_PAIR);
   hipError_t e = hipMalloc(&h->ws, sizeof(unsigned long long) * h->ws_words);
