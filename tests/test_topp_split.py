@@ -193,7 +193,8 @@ def test_topk_rows(sampler, oracle, V, bf16, mask, hist):
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 @pytest.mark.parametrize("rows,V,bf16,mask,chunks", [
     ([0, 1, 2, 3, 4, 5, 6, 7], 4097, False, False, 1), ([0, 8, 9, 10, 11, 12, 13], 4099, True, True, 1),
-    ([1, 9, 11, 13], 8192, True, False, 2), ([0, 3, 10], 16383, False, False, 3), ([2, 4, 8, 12], 12289, True, True, 3)])
+    ([1, 9, 11, 13], 8192, True, False, 2), ([0, 3, 10], 16383, False, False, 3), ([2, 4, 8, 12], 12289, True, True, 3),
+    ([0, 1, 2, 3, 4, 5, 6, 8, 9], 8200, False, False, 2)])
 def test_short_rows_in_the_simulation(oracle, rows, V, bf16, mask, chunks):
     """Rows that one workgroup's registers could hold, batches of every kind:
     one chunk or a few."""

@@ -28,8 +28,8 @@
 // No wait depends on a workgroup that has not started: the polls of steps 1
 // and 3 are bounded, and the owner waits only for workgroups that have
 // arrived, whose polls are bounded.  So any grid is safe, whatever else runs
-// on the device; rows are consecutive workgroups, so a row's chunks run
-// together.
+// on the device; the rows of a group of 8 are consecutive workgroups, so a row's
+// chunks run together.
 //
 // The exchange uses agent-scope loads and stores throughout (they pass the
 // per-XCD L2s, which are not coherent with each other) and plain waits for
@@ -288,7 +288,15 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   using RV = RowView<Tin, true, SBT>;
   using SV = RowView<Tin, false, SBT>;
   constexpr int NPRE = RV::NV < TOPP_MASK_PRE ? RV::NV : TOPP_MASK_PRE;
-  const int lb = (int)blockIdx.x / a.S, c = (int)blockIdx.x % a.S;
+  // Workgroups are dealt out to the 8 XCDs in turn: the rows of a group of 8
+  // alternate, so that a row's chunks share an XCD and the rows' owners (most
+  // often the last chunk's workgroup) are on all of them.  Row by row, with 8
+  // chunks, nearly all owners were on one XCD: 300 rows of 128,256 fp32 with
+  // k up to 1024 under masks of one chunk's ids took 276 us, now 179; with k
+  // above 1024 (the owner reads the row many times) 4845 and 2837.
+  const int g0 = (int)blockIdx.x / (8 * a.S) * 8, p8 = (int)blockIdx.x - g0 * a.S;
+  const int g = min(8, (int)gridDim.x / a.S - g0);
+  const int lb = g0 + p8 % g, c = p8 / g;
   const int b = a.row0 + lb;
   if (b >= a.B) return;
   const int w = threadIdx.x >> 6, lane = lane_id();
