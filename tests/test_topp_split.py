@@ -214,6 +214,43 @@ def test_short_rows_in_the_simulation(oracle, rows, V, bf16, mask, chunks):
             np.testing.assert_array_equal(r["ids"], o["ids"])
 
 
+def _large_k_rows(oracle, V, seed):
+    """Rows with 1024 < top_k < V whose sets end inside buckets of a few, of
+    many and of nearly all ids; top-p on, off and near zero."""
+    g = np.random.default_rng(seed)
+    x = np.concatenate([np.round(g.standard_normal((3, V)) * 2.0), np.full((2, V), 0.75), g.standard_normal((4, V)) * 3.0])
+    x[4, ::3] = 0.74
+    B = len(x)
+    p = oracle.make_params(B, temperature=0.8, top_p=[0.9, 1.0, 0.5, 0.6, 1.0, 0.99, 1.0, 1e-9, 0.9])
+    p["top_k"] = [V // 2, 1100, V - 1, 3000, V // 2, V // 2, 3000, V // 3, 1025]
+    return x.astype(np.float32), p, (g.integers(0, 1 << 24, B) / (1 << 24)).astype(np.float32)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("rows,V,concurrent", [([0, 3, 5], 12289, True), ([1, 4, 6], 8200, True),
+                                               ([2, 7, 8], 8200, True), ([0, 1, 2, 3, 4, 5, 6, 7, 8], 4100, True),
+                                               ([0, 4, 6], 8200, False)])
+def test_large_k_in_the_simulation(oracle, rows, V, concurrent):
+    import sim as S
+
+    S.build()
+    x, p, u = (t[rows] for t in _large_k_rows(oracle, V, V))
+    r = S.run_sample(x, p, u, kept_cap=8, concurrent=concurrent,
+                     env_extra={"TGS_KEY_SPINS": "100000"} if concurrent else None)
+    assert [blk for _, blk in r["launches"]] == [512]
+    H.compare(r, oracle.sample_batch(x, p, u, kept_cap=8, want_post=True, nthreads=8), p, V, what="large k")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V", [4100, 12289, 50001, 128256])
+@pytest.mark.parametrize("copies", [1, 29])
+def test_large_k(sampler, oracle, V, copies):
+    x, p, u = (np.concatenate([t] * copies) for t in _large_k_rows(oracle, V, V))
+    o = oracle.sample_batch(x, p, u, kept_cap=8, want_post=False, nthreads=8)
+    H.log(f"case large k V={V} B={len(p)}")
+    H.compare(H.run_gpu(sampler, x, p, u, kept_cap=8, post=False), o, p, V, what="large k", check_post=False)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("V,bf16,mask,hist", [
     (4097, False, False, 64), (4104, True, True, 0), (7325, True, False, 64), (11008, False, True, 1000),

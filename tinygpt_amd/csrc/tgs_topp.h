@@ -318,6 +318,19 @@ __device__ __forceinline__ u64 select_list(const u64* L, unsigned n, float m, u6
   return x;
 }
 
+// Bucket bq's ids (at most CAPL) into tl.L, from the row.  Starts and ends
+// with a barrier.
+template <int BT, class View>
+__device__ __forceinline__ void gather_bucket(const View& rv, Tail& tl, int bq, Scratch<BT>& ts) {
+  const float m = tl.m;
+  if (threadIdx.x == 0) ts.ng = 0;
+  __syncthreads();
+  rv.each_stream([&](int id, float y) {
+    if (bucket::of(y, m) == bq) tl.L[atomicAdd(&ts.ng, 1u)] = comp_key(tg_key(y), id);
+  });
+  __syncthreads();
+}
+
 // The element of bucket bq whose within-bucket inclusive prefix first
 // reaches target (>= 1): its composite, the mass ahead of it in the bucket
 // and its rank there.  The bucket's members are gathered from the row; a
@@ -329,12 +342,7 @@ __device__ __forceinline__ u64 resolve_mass(const View& rv, Tail& tl, int bq, u6
   const float m = tl.m;
   const unsigned n = tl.CI[bq] - bucket::count_before(tl.CI, bq);
   if (n <= (unsigned)CAPL) {
-    if (threadIdx.x == 0) ts.ng = 0;
-    __syncthreads();
-    rv.each_stream([&](int id, float y) {
-      if (bucket::of(y, m) == bq) tl.L[atomicAdd(&ts.ng, 1u)] = comp_key(tg_key(y), id);
-    });
-    __syncthreads();
+    gather_bucket<BT>(rv, tl, bq, ts);
     return select_list<BT>(tl.L, n, m, target, before, rank, tl.R, tl.Q, ts, bs);
   }
   auto en = [&](auto f) {
@@ -343,6 +351,37 @@ __device__ __forceinline__ u64 resolve_mass(const View& rv, Tail& tl, int bq, u6
     });
   };
   return block_mass_select<BT>(en, target, bs, before, rank);
+}
+
+// The ik-th largest (1-based) of bucket bq's ids and the mass of the ik
+// largest; as resolve_mass.
+template <int BT, class View>
+__device__ __forceinline__ u64 resolve_count(const View& rv, Tail& tl, int bq, unsigned ik, u64* mass,
+                                             Scratch<BT>& ts, BlockScratch& bs) {
+  const float m = tl.m;
+  const unsigned n = tl.CI[bq] - bucket::count_before(tl.CI, bq);
+  if (n <= (unsigned)CAPL) {
+    gather_bucket<BT>(rv, tl, bq, ts);
+    u64 before;
+    unsigned rank;
+    const u64 x = select_list<BT, true>(tl.L, n, m, ik, &before, &rank, tl.R, tl.Q, ts, bs);
+    *mass = before + bucket::mass_c(x, m);
+    return x;
+  }
+  auto en = [&](auto f) {
+    rv.each_stream([&](int id, float y) {
+      if (bucket::of(y, m) == bq) f(comp_key(tg_key(y), id));
+    });
+  };
+  const u64 T = block_select_kth<u64, 64, BT>(en, ik, bs);
+  u64 S = 0, minc = ~0ull;
+  en([&](u64 x) {
+    if (x < T) return;
+    S += bucket::mass_c(x, m);
+    minc = x < minc ? x : minc;
+  });
+  *mass = block_sum<u64, BT>(S, ts.red64);
+  return ~block_max<u64, BT>(~minc, ts.red64b);
 }
 
 // Pass 2: every allowed id of the view into the count and exact-mass
@@ -630,12 +669,29 @@ __device__ __forceinline__ u64 pick_gathered(Plan& pl, float top_p, Tail& tl, Sc
   return select_list<BT>(tl.L, pl.na, m, target, &before, &rank, tl.R2, tl.Q2, ts, bs);
 }
 
-// The same without the one-gather guarantee: the cut, then the draw, each
-// bucket gathered from the view (or radix selected beyond CAPL ids).
+// The same without the one-gather guarantee: the top-k set's end (when it
+// lies inside a bucket), the cut, then the draw, each one's bucket gathered
+// from the view (or radix selected beyond CAPL ids): three passes over the
+// row.  (Radix selections over the whole row, for rows with a top-k, read it
+// about twenty times: 1024 rows of 128,256 fp32 ids with k above 1024 took
+// 9.6 ms.)
 template <int BT, class View>
-__device__ __forceinline__ u64 pick_resolved(Plan& pl, const View& rv, Tail& tl, Scratch<BT>& ts, BlockScratch& bs) {
+__device__ __forceinline__ u64 pick_resolved(Plan& pl, float top_p, const View& rv, Tail& tl, Scratch<BT>& ts,
+                                             BlockScratch& bs) {
   u64 before;
   unsigned rank;
+  if (pl.k_search) {
+    u64 mass;
+    const u64 last = resolve_count<BT>(rv, tl, pl.bp, pl.nv - bucket::count_before(tl.CI, pl.bp), &mass, ts, bs);
+    pl.S = bucket::mass_before(tl.MI, pl.bp) + mass;
+    if (pl.cut_last) {
+      pl.cutc = last;
+      pl.Sp = pl.S;
+    } else if (pl.cut_search) {
+      pl.P = mul_shr24(pl.S, (uint32_t)(top_p * 16777216.0f));
+      pl.bp = bucket::find_mass<BT>(tl.MI, pl.P, &ts.sel[0]);
+    }
+  }
   if (pl.cut_search) {
     pl.cutc = resolve_mass<BT>(rv, tl, pl.bp, pl.P - bucket::mass_before(tl.MI, pl.bp), &before, &rank, ts, bs);
     pl.Sp = bucket::mass_before(tl.MI, pl.bp) + before + bucket::mass_c(pl.cutc, tl.m);
@@ -684,50 +740,6 @@ __device__ __forceinline__ void write_kept(const SampleArgs& a, int b, const u64
     for (int i = threadIdx.x; i < a.dbg.kept_cap; i += BT)
       kp[i] = i < ntopp ? kept_prob(comp_y(sorted[i]), m, fs) : 0.0f;
   }
-}
-
-// The row settled without the lists, by radix selections over the view read
-// again for every digit: a top-k of kk elements out of more allowed ids, any
-// ties.
-template <int BT, class View>
-__device__ __forceinline__ u64 pick_streamed(Plan& pl, unsigned kk, const Row& r, const View& sv, u64 Mc, Tail& tl,
-                                             Scratch<BT>& ts, BlockScratch& bs) {
-  const float m = tl.m;
-  pl.uq = (uint32_t)(r.u * 16777216.0f);
-  const u64 T = block_select_kth<u64, 64, BT>(
-      [&](auto f) { sv.each([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, kk, bs);
-  auto each_kept = [&](auto f) {
-    sv.each([&](int id, float y) {
-      const u64 x = comp_key(tg_key(y), id);
-      if (x >= T) f(x, bucket::mass(y, m));
-    });
-  };
-  u64 S = 0, minc = ~0ull;
-  each_kept([&](u64 x, u64 q) {
-    S += q;
-    minc = x < minc ? x : minc;
-  });
-  S = block_sum<u64, BT>(S, ts.red64);
-  minc = ~block_max<u64, BT>(~minc, ts.red64b);
-  u64 before;
-  unsigned rank;
-  pl.nv = pl.ntopp = kk;
-  pl.S = pl.Sp = S;
-  pl.cutc = minc;
-  pl.k_search = pl.cut_last = true;  // the cut is settled
-  if (r.top_p < 1.0f) {
-    pl.P = mul_shr24(S, (uint32_t)(r.top_p * 16777216.0f));
-    if (pl.P == 0) {
-      pl.cutc = Mc;
-      pl.Sp = tg_q40(1.0f);
-      pl.ntopp = 1;
-    } else {
-      pl.cutc = block_mass_select<BT>(each_kept, pl.P, bs, &before, &rank);
-      pl.Sp = before + bucket::mass_c(pl.cutc, m);
-      pl.ntopp = rank + 1;
-    }
-  }
-  return block_mass_select<BT>(each_kept, mul_shr24(pl.Sp, pl.uq) + 1, bs, &before, &rank);
 }
 
 // A greedy row (the largest composite Mc), or a row with nothing allowed

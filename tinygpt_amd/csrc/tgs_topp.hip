@@ -54,7 +54,7 @@ __device__ __forceinline__ void topp_rest(const SampleArgs& a, const Row& r, con
     __syncthreads();
     pick = pick_gathered<BT>(pl, r.top_p, tl, ts, bs);
   } else {
-    pick = pick_resolved<BT>(pl, rv, tl, ts, bs);
+    pick = pick_resolved<BT>(pl, r.top_p, rv, tl, ts, bs);
   }
   write_row<BT>(a, r.b, pl, pick, rv, ts);
 }

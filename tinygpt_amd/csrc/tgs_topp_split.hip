@@ -715,11 +715,7 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       __syncthreads();
       pick = pick_gathered<SBT>(pl, r.top_p, tl, sh.ts, sh.bs);
     } else {
-      if (!whole) {
-        pick = pick_streamed<SBT>(pl, kk, r, sv, Mc, tl, sh.ts, sh.bs);
-      } else {
-        pick = pick_resolved<SBT>(pl, sv, tl, sh.ts, sh.bs);
-      }
+      pick = pick_resolved<SBT>(pl, r.top_p, sv, tl, sh.ts, sh.bs);
     }
     if (kk < nall && whole && pl.cut_last && a.dbg.cut_ids) {
       const u64 T = block_select_kth<u64, 64, SBT>(
