@@ -399,12 +399,15 @@ __device__ __forceinline__ T block_max(T x, T* red) {
 // equals the kth largest key, or a prefix of it with zeroed low bits when
 // the keys of that prefix number exactly what is needed (then
 // #{key >= T} == kth).  kth >= 1 and the multiset holds >= kth keys.
+// The first digit starts at bit `shift`, below the bits pmask that every key is
+// known to share with prefix.
 template <typename K, int NBITS, int BS = NT, class Enum>
-__device__ __forceinline__ K block_select_kth(Enum en, unsigned kth, BlockScratch& s) {
-  K prefix = 0, pmask = 0;
+__device__ __forceinline__ K block_select_kth(Enum en, unsigned kth, BlockScratch& s, int shift = NBITS - 8,
+                                              K prefix = 0, K pmask = 0) {
   unsigned need = kth;
 #pragma unroll 1  // one pass live at a time: callers hold large register state across
-  for (int shift = NBITS - 8; shift >= 0; shift -= 8) {
+  for (;; shift -= 8) {
+    if (shift < 0) shift = 0;  // the last digit overlaps the one before it
     for (int i = threadIdx.x; i < 256; i += BS) s.hc[i] = 0;
     __syncthreads();
     en([&](K x) {
@@ -443,7 +446,7 @@ __device__ __forceinline__ K block_select_kth(Enum en, unsigned kth, BlockScratc
     const unsigned bc = (unsigned)s.binc_i;
     prefix |= (K)d << shift;
     pmask |= (K)255 << shift;
-    if (bc == need) break;
+    if (bc == need || shift == 0) break;
   }
   return prefix;
 }
@@ -497,15 +500,16 @@ __device__ __forceinline__ void mass_digit_scan(BlockScratch& s, u64 target, u64
 // `en(f)` calls f(key, mass) for every key this thread owns.  Returns the
 // element's key; *before gets the mass strictly ahead of it, *rank the
 // number of elements strictly ahead of it.
+// shift, prefix and pmask as for block_select_kth.
 template <int BS = NT, class Enum>
 __device__ __forceinline__ u64 block_mass_select(Enum en, u64 target, BlockScratch& s, u64* before,
-                                 unsigned* rank) {
-  u64 prefix = 0, pmask = 0;
+                                 unsigned* rank, int shift = 56, u64 prefix = 0, u64 pmask = 0) {
   u64 mass_above = 0;
   unsigned cnt_above = 0;
   bool single = false;
 #pragma unroll 1
-  for (int shift = 56; shift >= 0; shift -= 8) {
+  for (;; shift -= 8) {
+    if (shift < 0) shift = 0;
     for (int i = threadIdx.x; i < 256; i += BS) {
       s.hc[i] = 0;
       s.hm[i] = 0;
@@ -527,8 +531,8 @@ __device__ __forceinline__ u64 block_mass_select(Enum en, u64 target, BlockScrat
     const int bc = s.binc_i;
     prefix |= (u64)d << shift;
     pmask |= (u64)255 << shift;
-    if (bc == 1) {
-      single = shift > 0;
+    if (bc == 1 || shift == 0) {
+      single = bc == 1 && shift > 0;
       break;
     }
   }

@@ -318,6 +318,44 @@ __device__ __forceinline__ u64 select_list(const u64* L, unsigned n, float m, u6
   return x;
 }
 
+// The bits that the composites en(f) enumerates share, and where the first
+// digit that tells them apart starts (block_select_kth).  The ids of a
+// crowded bucket agree in most of their keys' bits, and a digit in which they
+// agree costs a pass whose LDS atomics all go to one bin: 64 top-p rows of
+// 128,256 equal fp32 logits took 5.9 ms from bit 63 down.
+struct Digits {
+  u64 prefix, pmask;
+  int shift;
+};
+template <int BT, class Enum>
+__device__ __forceinline__ Digits shared_digits(Enum en, Scratch<BT>& ts) {
+  u64 any = 0, all = ~0ull;
+  en([&](u64 x) {
+    any |= x;
+    all &= x;
+  });
+  any = wave_or64(any);
+  all = ~wave_or64(~all);
+  __syncthreads();
+  if (lane_id() == 0) {
+    ts.red64[threadIdx.x >> 6] = any;
+    ts.red64b[threadIdx.x >> 6] = all;
+  }
+  __syncthreads();
+  any = 0;
+  all = ~0ull;
+#pragma unroll
+  for (int v = 0; v < BT / 64; v++) {
+    any |= ts.red64[v];
+    all &= ts.red64b[v];
+  }
+  const u64 d = any ^ all;
+  if (d == 0ull) return Digits{all, ~0ull, 0};  // one composite
+  const int h = 63 - __clzll((long long)d);
+  const u64 pmask = h == 63 ? 0ull : ~0ull << (h + 1);
+  return Digits{all & pmask, pmask, h - 7};
+}
+
 // Bucket bq's ids (at most CAPL) into tl.L, from the row.  Starts and ends
 // with a barrier.
 template <int BT, class View>
@@ -345,12 +383,15 @@ __device__ __forceinline__ u64 resolve_mass(const View& rv, Tail& tl, int bq, u6
     gather_bucket<BT>(rv, tl, bq, ts);
     return select_list<BT>(tl.L, n, m, target, before, rank, tl.R, tl.Q, ts, bs);
   }
-  auto en = [&](auto f) {
+  auto each_of = [&](auto f) {
     rv.each_stream([&](int id, float y) {
-      if (bucket::of(y, m) == bq) f(comp_key(tg_key(y), id), bucket::mass(y, m));
+      if (bucket::of(y, m) == bq) f(id, y);
     });
   };
-  return block_mass_select<BT>(en, target, bs, before, rank);
+  const Digits d = shared_digits<BT>([&](auto f) { each_of([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, ts);
+  return block_mass_select<BT>(
+      [&](auto f) { each_of([&](int id, float y) { f(comp_key(tg_key(y), id), bucket::mass(y, m)); }); }, target, bs,
+      before, rank, d.shift, d.prefix, d.pmask);
 }
 
 // The ik-th largest (1-based) of bucket bq's ids and the mass of the ik
@@ -373,7 +414,8 @@ __device__ __forceinline__ u64 resolve_count(const View& rv, Tail& tl, int bq, u
       if (bucket::of(y, m) == bq) f(comp_key(tg_key(y), id));
     });
   };
-  const u64 T = block_select_kth<u64, 64, BT>(en, ik, bs);
+  const Digits d = shared_digits<BT>(en, ts);
+  const u64 T = block_select_kth<u64, 64, BT>(en, ik, bs, d.shift, d.prefix, d.pmask);
   u64 S = 0, minc = ~0ull;
   en([&](u64 x) {
     if (x < T) return;
@@ -580,21 +622,29 @@ __device__ __forceinline__ void gather(const RowView<Tin, true, BT>& rv, const P
     else sink(1, ob++, x);
   }
 }
-// The allowed ids with y >= yb, in no particular order (sink(place,
-// composite)); ts.ng counts them (zero before).  The same marks and places.
-template <typename Tin, int BT, class F>
-__device__ __forceinline__ void gather_floor(const RowView<Tin, true, BT>& rv, float yb, Scratch<BT>& ts, F sink) {
-  constexpr int EPV = Elem<Tin>::EPV;
+// The thread's slots that hold an allowed id with y >= yb, a bit each.
+template <typename Tin, int BT>
+__device__ __forceinline__ uint32_t floor_marks(const RowView<Tin, true, BT>& rv, float yb) {
   uint32_t ma = 0u;
 #pragma unroll
   for (int q = 0; q < RES_EPT; q++) ma |= (rv.y[q] >= yb && rv.y[q] > -__builtin_inff()) ? 1u << q : 0u;
+  return ma;
+}
+// Places for the marked slots of the wave's threads (the first of this
+// thread's): one wave scan and one LDS atomic; ts.ng counts them.
+template <int BT>
+__device__ __forceinline__ unsigned mark_places(uint32_t ma, Scratch<BT>& ts) {
   const unsigned n = (unsigned)__popc(ma);
   const unsigned incl = wave_incl_scan(n);
   const unsigned tot = readlane_u32(incl, 63);
-  if (tot == 0u) return;
   unsigned at = 0u;
-  if (lane_id() == 0) at = atomicAdd(&ts.ng, tot);
-  at = readlane_u32(at, 0) + incl - n;
+  if (lane_id() == 0 && tot) at = atomicAdd(&ts.ng, tot);
+  return readlane_u32(at, 0) + incl - n;
+}
+// sink(place, composite) for the marked slots.
+template <typename Tin, int BT, class F>
+__device__ __forceinline__ void each_marked(const RowView<Tin, true, BT>& rv, uint32_t ma, unsigned at, F sink) {
+  constexpr int EPV = Elem<Tin>::EPV;
 #pragma unroll
   for (int q = 0; q < RES_EPT; q++)
     if ((ma >> q) & 1u)
@@ -796,6 +846,19 @@ __device__ __forceinline__ u64 thread_best(const RowView<Tin, true, BT>& rv) {
   }
   const int mid = rv.r.v0 + ((int)threadIdx.x + (mq / EPV) * BT) * EPV + mq % EPV;
   return mx > -__builtin_inff() ? comp_key(tg_key(mx), mid) : 0ull;
+}
+
+// The key of the thread's second largest id (0: fewer than two allowed).
+template <typename Tin, int BT>
+__device__ __forceinline__ uint32_t thread_second(const RowView<Tin, true, BT>& rv) {
+  float m1 = -__builtin_inff(), m2 = -__builtin_inff();
+#pragma unroll
+  for (int q = 0; q < RES_EPT; q++) {
+    const float y = rv.y[q];
+    m2 = fmaxf(m2, fminf(m1, y));
+    m1 = fmaxf(m1, y);
+  }
+  return m2 > -__builtin_inff() ? tg_key(m2) : 0u;
 }
 
 }  // namespace topp

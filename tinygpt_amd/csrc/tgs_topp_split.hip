@@ -263,6 +263,78 @@ __device__ __forceinline__ float counted_floor(const RowView<Tin, true, SBT>& rv
   return m - (float)(q + 2) * 0.03125f;
 }
 
+// The slots of a chunk's k largest composites, a bit each (floor_marks); the
+// chunk holds at least k ids with y >= yb.  From its registers by bisection:
+// first over the keys, until exactly k ids are at or above the middle, then,
+// where several ids share the k-th key, over their ids.  mc: the thread's
+// largest composite.  At most 32 and 18 rounds of one barrier each; radix
+// digits over the chunk read again sent ties to one LDS bin (1 row of 128,256
+// equal fp32 logits, k = 1000: 376 us).  ts.ng is 0 after it; starts and ends
+// with a barrier.
+template <typename Tin>
+__device__ __forceinline__ uint32_t kth_marks(const RowView<Tin, true, SBT>& rv, u64 mc, unsigned k, float yb,
+                                              SplitShared& sh) {
+  constexpr int EPV = Elem<Tin>::EPV;
+  const int w = threadIdx.x >> 6;
+  unsigned turn = 0;
+  // the workgroup's sum of n (two sets of words in turn: one barrier)
+  auto sum = [&](unsigned n) -> unsigned {
+    n = wave_sum(n);
+    uint32_t* words = sh.wkey[turn & 1u][0];
+    turn++;
+    if (lane_id() == 0) words[w] = n;
+    __syncthreads();
+    n = 0;
+#pragma unroll
+    for (int v = 0; v < SBT / 64; v++) n += words[v];
+    return n;
+  };
+  const uint32_t mx = (uint32_t)(block_reduce_max<SBT>(mc, sh.ts.red64) >> 32);
+  if (threadIdx.x == 0) sh.ts.ng = 0;
+  // the largest key with k ids at or above it: in [lo, hi)
+  uint32_t lo = yb > -__builtin_inff() ? tg_key(yb) : 0x00800000u, hi = mx + 1u;
+  unsigned above = 0;  // ids at or above hi
+  bool met = false;    // exactly k ids at or above lo
+  while (hi - lo > 1u && !met) {
+    const uint32_t mid = lo + (hi - lo) / 2u;
+    const float ym = tg_unkey(mid);
+    unsigned n = 0;
+#pragma unroll
+    for (int q = 0; q < RES_EPT; q++) n += rv.y[q] >= ym ? 1u : 0u;
+    n = sum(n);
+    if (n >= k) {
+      lo = mid;
+      met = n == k;
+    } else {
+      hi = mid;
+      above = n;
+    }
+  }
+  const float yk = tg_unkey(lo);
+  uint32_t gt = 0u, eq = 0u;
+#pragma unroll
+  for (int q = 0; q < RES_EPT; q++) {
+    gt |= rv.y[q] > yk ? 1u << q : 0u;
+    eq |= rv.y[q] == yk ? 1u << q : 0u;
+  }
+  // the least offset in the chunk up to which the ids of that key make up the
+  // rest, in (a, z]: a thread's offsets rise with the slot
+  int a = -1, z = rv.r.v1 - rv.r.v0 - 1;
+  auto upto = [&](int last) -> uint32_t {
+    const int o = last - (int)threadIdx.x * EPV;  // slot q: offset (q / EPV) SBT EPV + q % EPV
+    if (o < 0) return 0u;
+    const int n = o / (SBT * EPV) * EPV + min(o % (SBT * EPV) + 1, EPV);
+    return n >= 32 ? eq : eq & ((1u << n) - 1u);
+  };
+  while (z - a > 1 && !met) {
+    const int mid = a + (z - a) / 2;
+    if (above + sum((unsigned)__popc(upto(mid))) >= k) z = mid;
+    else a = mid;
+  }
+  __syncthreads();
+  return gt | upto(z);
+}
+
 // The decision word: the epoch's low 24 bits over the list buckets in 40
 // (bit 0: they are to be gathered; a run of 512 buckets or more for list B is
 // settled by the owner alone).  Every ending of a row leaves the word with
@@ -373,17 +445,23 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   if (r.mode == 1 && !hist_k) {
     // ---- a top-k of at most KMAX: the chunk's ids that reach a floor under
     // the row's k-th largest y, and no more meetings.  Floors from the thread
-    // maxima (bound_key): the chunk's own k-th largest (k <= SBT), or, when S
-    // lists of that many would be too long (meet), the lowest over the chunks
-    // of each one's ceil(k / S)-th largest, or the highest of their k-th.
+    // maxima (bound_key): the chunk's own k-th largest, or, when S lists of
+    // that many would be too long (meet), the lowest over the chunks of each
+    // one's ceil(k / S)-th largest, or the highest of their k-th (the better one
+    // where a mask or an order leaves the row's largest ids to few chunks).
     const bool counted = a.S == 1 && 4 * r.k > 3 * SBT;
     const bool meet = a.S > 1 && (2 * a.S * r.k > CAPL || 2 * r.k > SBT);
     const int k2 = (r.k + a.S - 1) / a.S;
+    // (k > SBT: the ceil(k / 2)-th largest of the threads' second maxima has k
+    // ids at or above it)
+    const bool two = r.k > SBT;
+    const int k1 = two ? (r.k + 1) / 2 : r.k;
     const uint32_t srt = wave_sort_desc((uint32_t)(mc >> 32));
+    const uint32_t srt1 = two ? wave_sort_desc(thread_second(rv)) : srt;
 #pragma unroll
     for (int q = 1; q <= SBT / 64; q++) {
-      const int at = (r.k + q - 1) / q - 1, at2 = (k2 + q - 1) / q - 1;
-      const uint32_t x = readlane_u32(srt, at & 63), x2 = readlane_u32(srt, at2 & 63);
+      const int at = (k1 + q - 1) / q - 1, at2 = (k2 + q - 1) / q - 1;
+      const uint32_t x = readlane_u32(srt1, at & 63), x2 = readlane_u32(srt, at2 & 63);
       if (lane == 0) {
         sh.wkey[0][q - 1][w] = at < 64 ? x : 0u;
         sh.wkey[1][q - 1][w] = at2 < 64 ? x2 : 0u;
@@ -405,28 +483,20 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
     }
     float yb = kb ? tg_unkey(kb) : -__builtin_inff();
     if (counted) yb = counted_floor<Tin>(rv, mc, (unsigned)r.k, tl, sh);
-    gather_floor(rv, yb, sh.ts, [&](unsigned o, u64 x) {
-      if (o < (unsigned)TOPPS_PAIR) st(slab + o, x);
-    });
-    wait_stores();
+    uint32_t ma = floor_marks(rv, yb);
+    unsigned at = mark_places(ma, sh.ts);
     __syncthreads();
     unsigned n = sh.ts.ng;
     if (n > (unsigned)TOPPS_PAIR) {
       // more ids than the list holds (ties at the floor, no floor): the
-      // chunk's exact top k, read again
-      const SV cv(a, rc, hash, hbits, rowp);
-      const u64 T = block_select_kth<u64, 64, SBT>(
-          [&](auto f) { cv.each([&](int id, float y) { f(comp_key(tg_key(y), id)); }); }, (unsigned)r.k, sh.bs);
-      if (threadIdx.x == 0) sh.ts.ng = 0;
-      __syncthreads();
-      cv.each([&](int id, float y) {
-        const u64 x = comp_key(tg_key(y), id);
-        if (x >= T) st(slab + atomicAdd(&sh.ts.ng, 1u), x);
-      });
-      wait_stores();
-      __syncthreads();
-      n = sh.ts.ng;
+      // chunk's exact top k
+      ma = kth_marks(rv, mc, (unsigned)r.k, yb, sh);
+      at = mark_places(ma, sh.ts);
+      n = (unsigned)r.k;
     }
+    each_marked(rv, ma, at, [&](unsigned o, u64 x) { st(slab + o, x); });
+    wait_stores();
+    __syncthreads();
     if (threadIdx.x == 0) {
       st(done + c, ((u64)ep << 32) | n);
       wait_stores();
