@@ -531,12 +531,32 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
       if (n <= (unsigned)CAPL) {
         each_entry([&](unsigned i, u64 x) { tl.L[i] = x; });
       } else {
-        // (ties again: the row's top k out of the lists)
-        const u64 T = block_select_kth<u64, 64, SBT>([&](auto f) { each_entry([&](unsigned, u64 x) { f(x); }); },
-                                                     (unsigned)r.k, sh.bs);
+        // (ties again: the row's top k out of the lists)  The lists are long
+        // and many passes follow: a list per group of threads, eight entries'
+        // loads in flight (through each_entry 1 row of 128,256 equal fp32
+        // logits, k = 1000, took 317 us).
+        int per = SBT;  // threads per list
+        while (per * a.S > SBT) per >>= 1;
+        const int lc = (int)threadIdx.x / per;
+        const unsigned ln = lc < a.S ? sh.done[lc] - (lc ? sh.done[lc - 1] : 0u) : 0u;
+        const u64* list = slabs + (long long)lc * TOPPS_PAIR;
+        auto en = [&](auto f) {
+          constexpr int FLY = 8;
+#pragma unroll 1
+          for (unsigned i0 = threadIdx.x % (unsigned)per; i0 < ln; i0 += FLY * per) {
+            u64 x[FLY];
+#pragma unroll
+            for (int j = 0; j < FLY; j++) x[j] = i0 + j * per < ln ? ld(list + i0 + j * per) : 0ull;
+#pragma unroll
+            for (int j = 0; j < FLY; j++)
+              if (x[j]) f(x[j]);
+          }
+        };
+        const Digits d = shared_digits<SBT>(en, sh.ts);
+        const u64 T = block_select_kth<u64, 64, SBT>(en, (unsigned)r.k, sh.bs, d.shift, d.prefix, d.pmask);
         if (threadIdx.x == 0) sh.ts.ng = 0;
         __syncthreads();
-        each_entry([&](unsigned, u64 x) {
+        en([&](u64 x) {
           if (x >= T) tl.L[atomicAdd(&sh.ts.ng, 1u)] = x;
         });
         n = (unsigned)r.k;
