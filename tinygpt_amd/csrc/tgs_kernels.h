@@ -95,7 +95,8 @@ struct SampleArgs {
   int hint_k;            // the launch hint's max_top_k (INT_MAX without a hint)
   int topp_all;          // 1: the top-p kernel alone serves the batch (its greedy rows too)
   unsigned long long* tp_lines;  // split top-p kernel: [rows][TOPPS_LINE] exchange lines (zero at set-up)
-  int row0;              // split top-p kernel: the launch's first row (slabs are indexed from it)
+  int row0, rows;        // split kernel: the launch's first row (slabs are indexed from it) and its rows
+  unsigned div8s, divg;  // and the multipliers that divide by 8 S and by the rows past the last group of 8
   int topp_cap;          // top-p kernel: allowed ids packed into LDS (beyond topp_lds_bytes)
   tgs_debug dbg;
 };

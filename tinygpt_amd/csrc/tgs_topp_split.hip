@@ -46,6 +46,8 @@
 // id), slabs out and counted 13.8, slabs summed 16.0, decision 17.6, lists in
 // 23.2, row written 25.5.  Chunks: at most 16384 ids (32 per thread; more
 // spill), about one workgroup per CU, at least 4096 ids.
+#include <algorithm>
+
 #include "tgs_topp.h"
 
 namespace tgs {
@@ -366,9 +368,12 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   // chunks, nearly all owners were on one XCD: 300 rows of 128,256 fp32 with
   // k up to 1024 under masks of one chunk's ids took 276 us, now 179; with k
   // above 1024 (the owner reads the row many times) 4845 and 2837.
-  const int g0 = (int)blockIdx.x / (8 * a.S) * 8, p8 = (int)blockIdx.x - g0 * a.S;
-  const int g = min(8, (int)gridDim.x / a.S - g0);
-  const int lb = g0 + p8 % g, c = p8 / g;
+  // (The divisions by 8 S and by the last group's rows are multiplications:
+  // one integer division is 40 dependent operations ahead of the first load.)
+  const int g0 = (int)__umulhi(blockIdx.x, a.div8s) * 8, p8 = (int)blockIdx.x - g0 * a.S;
+  const bool full = g0 + 8 <= a.rows;
+  const int c = full ? p8 >> 3 : (int)((unsigned)p8 * a.divg >> 16);
+  const int lb = g0 + p8 - c * (full ? 8 : a.rows - g0);
   const int b = a.row0 + lb;
   if (b >= a.B) return;
   const int w = threadIdx.x >> 6, lane = lane_id();
@@ -828,7 +833,10 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
 hipError_t launch_topps(SampleArgs a, int dtype, int rows, hipStream_t st) {
   const size_t lds = topp_lds_bytes(a.V, a.TS);
   for (a.row0 = 0; a.row0 < a.B; a.row0 += rows) {
-    const dim3 g((unsigned)((rows < a.B - a.row0 ? rows : a.B - a.row0) * a.S)), blk(TOPPS_NT);
+    a.rows = rows < a.B - a.row0 ? rows : a.B - a.row0;
+    a.div8s = (unsigned)((1ull << 32) / (unsigned)(8 * a.S) + 1);  // exact below 2^32 / (8 S)
+    a.divg = 65536u / (unsigned)std::max(a.rows % 8, 1) + 1u;       // exact below 2^16 / g
+    const dim3 g((unsigned)(a.rows * a.S)), blk(TOPPS_NT);
     if (dtype == 1) hipLaunchKernelGGL((topp::topps_kernel<uint16_t>), g, blk, lds, st, a);
     else hipLaunchKernelGGL((topp::topps_kernel<float>), g, blk, lds, st, a);
     const hipError_t e = hipGetLastError();
