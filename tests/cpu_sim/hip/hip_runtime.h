@@ -133,8 +133,16 @@ inline BlockCtx*& block_ctx() { return t_ctx; }
 inline thread_local dim3 t_thread, t_block;
 inline dim3 g_block_dim, g_grid_dim;
 inline unsigned char* dyn_smem() { return block_ctx()->smem.data(); }
+// LDS of the simulated device (TGS_SIM_LDS: a smaller one).
+inline size_t lds_limit() {
+  static const size_t n = std::getenv("TGS_SIM_LDS") ? (size_t)std::atoll(std::getenv("TGS_SIM_LDS")) : 163840;
+  return n;
+}
 inline unsigned char* static_smem(size_t n) {
-  if (n > kStaticSmem) std::abort();
+  if (n > kStaticSmem || n + block_ctx()->smem.size() > lds_limit()) {
+    std::fprintf(stderr, "static and dynamic LDS beyond the device's: %zu + %zu\n", n, block_ctx()->smem.size());
+    std::abort();
+  }
   return block_ctx()->ssmem.data();
 }
 
@@ -433,7 +441,7 @@ inline hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipGetDeviceCount(int* n) { *n = 1; return hipSuccess; }
 inline hipError_t hipDeviceGetAttribute(int* v, int attr, int) {
-  *v = attr == hipDeviceAttributeMultiprocessorCount ? 256 : 163840;
+  *v = attr == hipDeviceAttributeMultiprocessorCount ? 256 : (int)hipcpu::lds_limit();
   return hipSuccess;
 }
 inline hipError_t hipFuncSetAttribute(const void*, int, int) { return hipSuccess; }

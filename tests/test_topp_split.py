@@ -214,6 +214,31 @@ def test_short_rows_in_the_simulation(oracle, rows, V, bf16, mask, chunks):
             np.testing.assert_array_equal(r["ids"], o["ids"])
 
 
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("top_k", [0, 2000])
+def test_rows_that_lds_does_not_hold(oracle, top_k):
+    """A device whose LDS holds the top-p kernel's tail but not the split
+    kernel's: rows beyond one workgroup's registers are refused before
+    anything is launched, shorter ones go to the kernels that fit."""
+    import sim as S
+
+    import tinygpt_amd as tg
+
+    S.build()
+    g = np.random.default_rng(44)
+    for V in (33000, 8000):
+        x = (g.standard_normal((1, V)) * 3.0).astype(np.float32)
+        p = oracle.make_params(1, temperature=0.8, top_k=top_k, top_p=0.9)
+        u = np.full(1, 0.5, np.float32)
+        run = lambda hint: S.run_sample(x, p, u, post=False, kept_cap=8, hint=hint, env_extra={"TGS_SIM_LDS": "44000"})  # noqa: E731
+        for hint in (tg.batch_hint(p, V), None):
+            if V == 33000:
+                with pytest.raises(RuntimeError, match=r"sample -5 .*\(top-p rows\)"):
+                    run(hint)
+            else:
+                np.testing.assert_array_equal(run(hint)["ids"], oracle.sample_batch(x, p, u)["ids"])
+
+
 def _large_k_rows(oracle, V, seed):
     """Rows with 1024 < top_k < V whose sets end inside buckets of a few, of
     many and of nearly all ids; top-p on, off and near zero."""

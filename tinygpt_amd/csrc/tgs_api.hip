@@ -382,16 +382,23 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
     return TGS_OK;
   }
   const int mink = hint ? hint->min_top_k : 0;
-  if (mk >= V && mink >= V && tgs::topp_lds_bytes(V, a.TS) + 2 * sizeof(tgs::BlockScratch) <= res.lds_limit) {
-    // every sampling row without a usable top-k: the top-p kernel serves the
+  // a row without a top-k: the top-p kernel holds one of up to
+  // topp_resident_ids() ids, the split kernel any; each with its own static LDS
+  const size_t tail_lds = tgs::topp_lds_bytes(V, a.TS);
+  const bool long_rows = V > tgs::topp_resident_ids();
+  const bool split_fits = tail_lds + tgs::topps_static_lds() + 256 <= res.lds_limit;
+  const bool topp_fits = long_rows ? split_fits : tail_lds + 2 * sizeof(tgs::BlockScratch) <= res.lds_limit;
+  if (mk >= V && mink >= V && topp_fits) {
+    // every sampling row without a usable top-k: one of the two serves the
     // batch alone, greedy rows included
     a.full_rows = 1;
     a.topp_all = 1;
-    return topp_core(res, err, a, dt, V > tgs::topp_resident_ids(), stream);
+    return topp_core(res, err, a, dt, long_rows, stream);
   }
   a.full_rows = (mk > tgs::KMAX || mk >= V) ? 1 : 0;
-  if (split_takes(res.num_cu, B, V) && tgs::topp_lds_bytes(V, a.TS) + tgs::topps_static_lds() + 256 <= res.lds_limit)
-    return topp_core(res, err, a, dt, true, stream);
+  if (split_takes(res.num_cu, B, V) && split_fits) return topp_core(res, err, a, dt, true, stream);
+  if (a.full_rows && (long_rows || !topp_fits))
+    return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS (top-p rows)");
   const int S = choose_split(res.num_cu, res.ws_rows, B, V);
   const int L = S > 1 ? ((V + S - 1) / S + 1023) / 1024 * 1024 : V;
   a.ws_stride = tgs::KMAX;
@@ -405,11 +412,9 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
   const size_t lds = (size_t)a.off_cand + (size_t)a.capt * 8;
   if (lds + sizeof(tgs::BlockScratch) > res.lds_limit)
     return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS");
-  if (a.full_rows && tgs::topp_lds_bytes(V, a.TS) + 2 * sizeof(tgs::BlockScratch) > res.lds_limit)
-    return efail(err, TGS_ETOOBIG, "history / vocab too large for LDS (top-p rows)");
   hipError_t e = tgs::launch_sample(a, dt, lds, stream);
   if (e != hipSuccess) return efail(err, TGS_EHIP, std::string("sample kernel launch: ") + hipGetErrorString(e));
-  return a.full_rows ? topp_core(res, err, a, dt, V > tgs::topp_resident_ids(), stream) : TGS_OK;
+  return a.full_rows ? topp_core(res, err, a, dt, false, stream) : TGS_OK;
 }
 
 // ---------------------------------------------------------------- allocation-free sampling
