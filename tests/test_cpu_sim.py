@@ -83,9 +83,26 @@ def test_chunk_kernel_waves_apart(sim, oracle):
     H.compare(r, o, params, V, what="sim")
 
 
+# a device whose LDS does not hold the split kernel: batches of every kind of
+# row go to the chunk, merge, full-path and top-p kernels at any length
+OLD_ROUTE = {"TGS_SIM_LDS": "44000"}
+
+
 def test_split_rows_and_merge(sim, oracle):
     x, params, u, hist, hist_len = _batch(13, 4, 5000, oracle)
-    _check(sim, oracle, x, params, u, hist, hist_len, split=3)
+    # no history: with one these rows' LDS goes past the limit too
+    r = sim.run_sample(x, params, u, kept_cap=1025, split=3, env_extra=OLD_ROUTE)
+    assert r["launches"] == [(12, 256), (4, 256), (4, 256), (4, 1024)]  # chunk, merge, full, top-p
+    o = oracle.sample_batch(x, params, u, kept_cap=1025, want_post=True)
+    H.compare(r, o, params, 5000, what="sim")
+
+
+@pytest.mark.parametrize("split", [1, 2, 3])
+def test_split_kernel_rows(sim, oracle, split):
+    """The same batch through the split kernel, over one to three chunks."""
+    x, params, u, hist, hist_len = _batch(13, 4, 5000, oracle)
+    r, _, _ = _check(sim, oracle, x, params, u, hist, hist_len, split=split)
+    assert r["launches"] == [(4 * split, 512)]
 
 
 def test_grammar_mask(sim, oracle):
@@ -173,7 +190,12 @@ def test_noalloc_entry_point(sim, oracle, path):
         _check(sim, oracle, x, params, u, hist, hist_len, mask=mask, hint=tg.batch_hint(params, V), split=4,
                kept_cap=64, noalloc=True)
     else:
-        _check(sim, oracle, x, params, u, hist, hist_len, mask=mask, split=2, noalloc=True)
+        r, _, _ = _check(sim, oracle, x, params, u, hist, hist_len, mask=mask, split=2, noalloc=True)
+        assert r["launches"][1:] == [(14, 512)]  # the split kernel (after the set-up fill)
+        r = sim.run_sample(x, params, u, mask_table=mask, kept_cap=1025, split=2, noalloc=True, env_extra=OLD_ROUTE)
+        assert r["launches"][1:] == [(14, 256), (7, 256), (7, 256), (7, 1024)]
+        H.compare(r, oracle.sample_batch(x, params, u, mask_table=mask, kept_cap=1025, want_post=True), params, V,
+                  what="sim")
 
 
 @pytest.mark.parametrize("split", [1, 3])
@@ -581,7 +603,12 @@ def test_topp_kernel_bucket_overflow(sim, oracle):
     params = oracle.make_params(B, temperature=1.0, top_k=0, top_p=0.37)
     params["top_p"][2] = 1.0
     u = np.array([0.1, 0.5, 0.99], np.float32)
-    _check(sim, oracle, x, params, u, None, None)
+    import tinygpt_amd as tg
+
+    r, _, _ = _check(sim, oracle, x, params, u, None, None, hint=tg.batch_hint(params, V))
+    assert r["launches"] == [(B, 1024)]  # the top-p kernel
+    r, _, _ = _check(sim, oracle, x, params, u, None, None)
+    assert r["launches"] == [(B, 512)]  # the split kernel, one chunk
 
 
 def test_topp_kernel_dense_rows_in_registers(sim, oracle):

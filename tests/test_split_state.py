@@ -90,3 +90,21 @@ def test_done_words_come_round(oracle):
     not taken for the current call's."""
     _run(oracle, [_call(oracle, "topp", seed=40), _call(oracle, "greedy", seed=41, epoch=(1 << 32) - 2),
                   _call(oracle, "topp", seed=42)])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B", [1, 9])
+def test_kinds_and_lengths_alternate_on_the_gpu(oracle, B):
+    """The same on the device, with up to 16 chunks per row."""
+    import gpu_harness as H
+    import tinygpt_amd as tg
+
+    s = tg.Sampler(device=0, max_batch=B, max_vocab=151936, max_hist=1)
+    kinds = ["topp", "list", "topp", "masked", "wide", "greedy", "topp", "invalid", "topp", "list", "masked", "topp"]
+    lengths = [128256, 50001, 8200, 128256, 151936, 4200, 33000, 128256, 50001, 16384, 151936, 128256]
+    for i, (kind, V) in enumerate(zip(kinds, lengths)):
+        c = _call(oracle, kind, V, B=B, seed=60 + i)
+        H.log(f"case split state call {i} {kind} V={V} B={B}")
+        r = H.run_gpu(s, c["x"], c["p"], c["u"], mask_table=_table(V), kept_cap=8, post=False)
+        np.testing.assert_array_equal(r["ids"], _ids(oracle, c), err_msg=f"call {i}")
+    s.close()

@@ -140,10 +140,11 @@ int choose_split(int num_cu, int ws_rows, int B, int V) {
   return S;
 }
 
-// Chunks per row of the split top-p kernel: about one workgroup per CU, at
-// least what its registers need, chunks of at least 4096 ids (below that the
-// row's exchanges outweigh the work a further chunk takes over), in slabs the
-// workspace holds.
+// Chunks per row of the split kernel: as many as keep the launch within one
+// workgroup per CU, of at least kSplitMin ids (below that the row's exchanges
+// outweigh the work a further chunk takes over), but at least what a chunk's
+// registers need, however many workgroups that makes (96 rows of 128,256: 768).
+// TGS_SPLIT sets the split (tuning, tests).
 constexpr int kSplitMin = 4096;  // least ids of a chunk
 // Slabs of a handle at most (15 KB each).  Each launch ends with the rows that
 // take longest alone on the chip: with 1024 slabs, 512 top-p rows of 151,936
@@ -153,8 +154,9 @@ constexpr int kSplitMin = 4096;  // least ids of a chunk
 constexpr int kSplitSlabs = 4096;
 int choose_split_topp(int num_cu, int B, int V) {
   const int smin = (V + tgs::TOPPS_CHUNK - 1) / tgs::TOPPS_CHUNK;
-  const int S = std::min({tgs::TOPPS_MAX_SPLIT, num_cu / std::max(B, 1), V / kSplitMin});
-  return std::max(S, smin);
+  const char* env = std::getenv("TGS_SPLIT");
+  const int want = env && std::atoi(env) > 0 ? std::atoi(env) : std::min(num_cu / std::max(B, 1), V / kSplitMin);
+  return std::max(std::min(want, tgs::TOPPS_MAX_SPLIT), smin);
 }
 
 // Whether the split kernel takes a batch of every kind of row: rows beyond one
