@@ -100,17 +100,19 @@ typedef struct {
 } tgs_debug;
 
 /* Host-side summary of a batch's row parameters.  It selects kernels
- * specialised for the batch: max_top_k <= 64 -> one-tile chunks merged in
- * wave registers (one launch); <= 1024 -> one workgroup per row holding the
- * row in registers (16-byte aligned rows of whole vectors: bf16 V <= 163840,
- * fp32 V <= 81920, history <= 1024 ids), else the candidate path; otherwise
- * (or no hint) the candidate path, the full-path kernel for rows with
- * 1024 < top_k < V and the top-p kernel for rows without a top-k.  The hint
- * is a promise: a sampling row whose top_k exceeds max_top_k (a row without
- * a usable top-k counts as V) gets id -3.  Greedy rows are served under any
- * hint.  min_top_k == V (every sampling row without a usable top-k, as in
- * grammar-constrained top-p decoding) lets the top-p kernel serve the whole
- * batch, its greedy rows included, in one launch. */
+ * specialised for the batch: max_top_k <= 64 -> the fused kernel (one launch;
+ * history <= 1024 ids); <= 1024 -> one workgroup per row holding the row in
+ * registers (16-byte aligned rows of whole vectors: bf16 V <= 163840, fp32
+ * V <= 81920, history <= 1024 ids); min_top_k == V (every sampling row without
+ * a usable top-k, as in grammar-constrained top-p decoding) -> one workgroup
+ * per row of at most 32768 ids, several per longer row, greedy rows included.
+ * Every other batch, and one without a hint, takes the split kernel from 4097
+ * ids on (every kind of row in one launch; not for 16385 to 32768 ids with
+ * more rows than the device has CUs), else the candidate kernels, the full-path
+ * kernel for rows with 1024 < top_k < V and the top-p kernel for rows without
+ * a top-k.  The hint is a promise: a sampling row whose top_k exceeds
+ * max_top_k (a row without a usable top-k counts as V) gets id -3.  Greedy
+ * rows are served under any hint. */
 typedef struct {
   int32_t max_top_k; /* max over sampling rows of top_k when 1 <= top_k < V, else V;
                         0 when every row is greedy */
@@ -171,7 +173,7 @@ int tgs_sample(tgs_handle h, const void* d_logits, tgs_dtype dt, int B, int V, i
  * samples inline in Swift/MLX.  Same arguments, kernels and results as
  * tgs_sample; the mask table is passed in (d_mask_table: n_states rows of
  * ceil(mask_vocab / 32) words, mask_vocab >= V; NULL / 0 for none).  Its
- * workspace is a static device array of about 6 MiB that every GPU the
+ * workspace is a static device array of about 18 MiB that every GPU the
  * library runs on holds until the process ends; the first call on a device
  * also prepares that array (and synchronises the device once), so it must
  * not be made under graph capture (it then returns TGS_EINVAL): make it

@@ -1,11 +1,11 @@
 // tgs_api.hip -- host side of the C ABI declared in include/tgs_sampler.h.
 //
-// The handle owns the split-row workspace (chunk candidate lists), the
-// speculative workspace and the mask table.  Calls validate host-visible
-// arguments, pick the kernel variant from the batch hint and the split
-// (chunks per row) from the batch size, size the dynamic LDS and launch on
-// the caller's stream (chunk kernel, then the merge kernel when rows are
-// split).  Nothing here allocates during tgs_sample.
+// The handle owns the workspace (chunk lists, split-kernel slabs, exchange
+// lines), the speculative workspace and the mask table.  Calls validate
+// host-visible arguments, pick the kernels from the batch hint and the sizes
+// (sample_core) and the chunks per row from the batch size, size the dynamic
+// LDS and launch on the caller's stream.  Nothing here allocates during
+// tgs_sample.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -162,10 +162,12 @@ int choose_split_topp(int num_cu, int B, int V) {
 // Whether the split kernel takes a batch of every kind of row: rows beyond one
 // workgroup's registers always; shorter ones of more than kSplitMin ids
 // instead of the chunk, merge, full-path and top-p launches (41 mixed rows of
-// 11,008 fp32 ids 75 -> 33 us, 1000 of 16,000 135 -> 61, 223 of 7,325 bf16 with
-// k up to 1024 56 -> 30). Rows of two chunks only while the launch stays
-// within two workgroups per CU: 200 mixed rows of 32,000 139 -> 54, but 500
-// top-p rows of 20,000 without a hint take 50 there and 47 by the old launches.
+// 11,008 fp32 ids 78 -> 32 us, 1000 of 16,000 138 -> 62, 223 of 7,325 bf16 with
+// k up to 1024 54 -> 30). Rows of two chunks only while the launch stays
+// within two workgroups per CU (200 mixed rows of 32,000 bf16 133 -> 51):
+// beyond, mixed batches would gain too (257 of 32,000 bf16 121 -> 51, 1000 214
+// -> 112), but batches of top-p rows that come without a hint lose (1000 of
+// 20,000 bf16 82 -> 93), and without one the two look alike.
 bool split_takes(int num_cu, int B, int V) {
   if (V <= kSplitMin || V > tgs::topp_resident_ids()) return V > kSplitMin;
   return V <= tgs::TOPPS_CHUNK || B <= num_cu;
@@ -228,9 +230,10 @@ int efail(std::string& err, int code, const std::string& msg) {
   return code;
 }
 
-// The rows without a top-k (all of a batch's, greedy rows too, with
-// a.topp_all): one workgroup per row where a row fits its registers, several
-// per row beyond.
+// split: the split kernel, for every row of the batch (with a.topp_all for
+// greedy rows and those without a top-k alone).  Otherwise the top-p kernel,
+// one workgroup per row, for the rows without a top-k (and with a.topp_all the
+// greedy ones).
 int topp_core(const SampleRes& res, std::string& err, tgs::SampleArgs a, tgs_dtype dt, bool split, hipStream_t stream) {
   hipError_t e;
   if (split) {
@@ -299,10 +302,12 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
   a.lists = res.k64_lists;
   a.keys = res.k64_keys;
   a.dbg = dz;
-  // Kernels: the fused top_k <= 64 kernel when the hint says every row is
-  // greedy or has top_k <= 64; otherwise the chunk kernel (+ merge kernel
-  // for split rows), plus the full-path kernel when the hint allows rows
-  // without a usable top-k.
+  // Kernels: every row greedy or top_k <= 64, the fused kernel; every row
+  // greedy or top_k <= KMAX and whole aligned vectors, the top-k kernel; every
+  // sampling row without a usable top-k, the top-p kernel, or the split kernel
+  // for long rows; any other batch the split kernel where split_takes says so,
+  // else the chunk kernel (+ merge kernel for split rows) and, when the hint
+  // allows rows without a top-k <= KMAX, the full-path and the top-p kernel.
   const int mk = hint ? hint->max_top_k : 0x7FFFFFFF;
   a.hint_k = mk;
   a.TS = hist_cap > 0 ? next_pow2(std::max(64, 2 * hist_cap)) : 0;

@@ -40,9 +40,10 @@ struct Scratch {
 
 // The canonical logits of ids [r.v0, r.v1) of a row (r.v0 a multiple of 32):
 // y after penalties and temperature, -inf where the id is not allowed (mask
-// bit clear, -inf or NaN).  RES: they fit in registers (RES_EPT ids per
-// thread, loaded once); otherwise every walk streams them again from L2 /
-// MALL.
+// bit clear, -inf or NaN).  RES: held in registers (RES_EPT ids per thread,
+// loaded once).  Otherwise every walk streams them again from L2 / MALL: the
+// fallback of a workgroup that finishes a row, or a partner's chunk, whose ids
+// it does not hold.
 template <typename Tin, bool RES, int BT>
 struct RowView {
   static constexpr int EPV = Elem<Tin>::EPV;

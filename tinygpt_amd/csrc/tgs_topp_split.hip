@@ -1,8 +1,8 @@
-// tgs_topp_split.hip -- rows that sample with top-p over a vocabulary too
-// long for one workgroup's registers (tgs_topp.hip holds those), each row
-// over S workgroups of 512 threads in one launch; in a launch that serves
-// the whole batch, the greedy rows too.  Batches of every kind of row come
-// here from 4,097 ids on; a row of one chunk skips the exchanges.
+// tgs_topp_split.hip -- every kind of row over S workgroups of 512 threads, in
+// one launch: rows without a top-k too long for one workgroup's registers
+// (tgs_topp.hip holds the others), with the batch's greedy rows where the hint
+// says so, and whole batches of every kind from 4,097 ids on (split_takes,
+// tgs_api.hip).  A row of one chunk skips the exchanges.
 //
 // What bounds it: one workgroup streams a row at one CU's rate and evaluates
 // every id's exact mass (about 40 VALU operations) on one CU, three passes
@@ -39,8 +39,8 @@
 // (reset_line).
 //
 // Measured against one workgroup per row streaming it three times (per call):
-// 1 row of 151,936 bf16 ids with penalties 137 -> 30 us, 32 rows of 128,256
-// fp32 ids 141 -> 28 us.  What bounds it now is the chain (stamps of the
+// 1 row of 151,936 bf16 ids with penalties 137 -> 31 us, 32 rows of 128,256
+// fp32 ids 141 -> 27 us.  What bounds it now is the chain (stamps of the
 // second, us from the first workgroup's entry): logits in registers 4.7,
 // row's maximum 7.1, histogram 12.1 (the exact exp and two LDS atomics per
 // id), slabs out and counted 13.8, slabs summed 16.0, decision 17.6, lists in
@@ -437,10 +437,10 @@ __global__ __launch_bounds__(SBT) void topps_kernel(SampleArgs a) {
   // a top-k past one wave's lists (of one chunk), or past what S short lists
   // hold, whose kept list nobody asked for goes through the histograms like a
   // larger one: the list's cut, mass and draw each select by digits, and lists
-  // beyond CAPL select the set first (223 rows of 7,325 bf16 ids, k up to 1024:
-  // 58 -> 30 us; 200 mixed rows of 32,000 109 -> 54).  Over more chunks the
-  // list has one meeting against three (41 mixed rows of 11,008: 29 by lists
-  // alone, 33 with this rule)
+  // beyond CAPL select the set first.  Lists alone, now that a chunk's exact top
+  // k is a bisection, are about level: 223 rows of 7,325 bf16 ids with k up to
+  // 1024 31.1 us (30.3 with this rule), 41 mixed rows of 11,008 fp32 35.4
+  // (32.0), 41 of 11,008 with k up to 1024 31.9 (35.2)
   const bool hist_k = r.k > (a.S == 1 ? 64 : 256 * a.S) && !a.dbg.kept_ids && !a.dbg.kept_probs;
   u64 mc = thread_best<Tin, SBT>(rv);
   u64* slab = a.ws + ((long long)lb * a.S + c) * TOPPS_PAIR;
