@@ -239,6 +239,65 @@ def test_rows_that_lds_does_not_hold(oracle, top_k):
                 np.testing.assert_array_equal(run(hint)["ids"], oracle.sample_batch(x, p, u)["ids"])
 
 
+def _floor_rows(oracle, V, seed, bf16):
+    """Rows that leave a floor below too many of a chunk's ids: in order, all
+    equal, all but one equal, of a few values around 0 of both signs, infinite
+    at more ids than k, and allowed in one stretch or at few ids only; and one
+    whose largest ids lie two to a thread of the first chunk, so that its k-th
+    is hardly above the floor."""
+    from tinygpt_amd import workloads as W
+
+    g = np.random.default_rng(seed)
+    n = np.sort(g.standard_normal(V) * 3.0)
+    x = np.stack([n, n[::-1], np.full(V, 0.75), np.full(V, -1e4), g.choice([-1e-40, -0.0, 0.0, 1e-40], V),
+                  g.standard_normal(V), g.standard_normal(V), g.standard_normal(V),
+                  g.uniform(-6.0, -5.0, V)]).astype(np.float32)
+    x[3, V // 3] = 5.0
+    first = np.arange(min(512, V // 16)) * (8 if bf16 else 4)
+    x[8, first], x[8, first + 1] = g.uniform(10.0, 11.0, len(first)), g.uniform(5.0, 6.0, len(first))
+    x[5, g.choice(V, V // 2, replace=False)] = np.inf
+    B, words = len(x), (V + 31) // 32
+    bits = np.zeros((2, words * 32), bool)
+    bits[0, V // 8:V // 3] = True
+    bits[1, g.choice(V, 600, replace=False)] = True
+    p = oracle.make_params(B, temperature=0.8, top_p=[0.9, 1.0, 0.5, 0.99, 0.9, 0.7, 0.95, 0.9, 1.0],
+                           mask_state=[-1, -1, -1, -1, -1, -1, 0, 1, -1])
+    p["top_k"] = [1000, 1024, 513, 700, 900, 600, 1023, 1000, 1000]
+    u = (g.integers(0, 1 << 24, B) / (1 << 24)).astype(np.float32)
+    return (W.f32_to_bf16_bits(x) if bf16 else x), p, u, np.packbits(bits, axis=1, bitorder="little").view(np.uint32)
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("rows,V,bf16,split,concurrent", [
+    ([0, 1, 2, 3, 4, 5, 6, 7], 4609, False, None, True), ([0, 2, 8], 12289, True, None, True),
+    ([1, 3, 8], 12289, False, None, True), ([4, 5], 8200, True, None, True), ([6, 7], 16384, False, 5, True), ([0, 4, 6], 8200, False, None, False)])
+def test_floors_in_the_simulation(oracle, rows, V, bf16, split, concurrent):
+    import sim as S
+
+    S.build()
+    x, p, u, table = _floor_rows(oracle, V, V, bf16)
+    x, p, u = x[rows], p[rows], u[rows]
+    r = S.run_sample(x, p, u, mask_table=table, kept_cap=1025, split=split, concurrent=concurrent,
+                     env_extra={"TGS_KEY_SPINS": "100000"} if concurrent else None)
+    assert [blk for _, blk in r["launches"]] == [512]
+    o = oracle.sample_batch(x, p, u, mask_table=table, kept_cap=1025, want_post=True, nthreads=8)
+    H.compare(r, o, p, V, what="floors")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("V,bf16", [(4609, True), (12289, False), (32000, True), (128256, False), (151935, True)])
+@pytest.mark.parametrize("copies", [1, 33])
+def test_floors(sampler, oracle, V, bf16, copies):
+    x, p, u, table = _floor_rows(oracle, V, V + 1, bf16)
+    o = oracle.sample_batch(x, p, u, mask_table=table, kept_cap=1025, want_post=False, nthreads=8)
+    rep = lambda t: np.concatenate([t] * copies)  # noqa: E731
+    H.log(f"case floors V={V} bf16={bf16} B={copies * len(p)}")
+    r = H.run_gpu(sampler, rep(x), rep(p), rep(u), mask_table=table, kept_cap=1025, post=False)
+    for i in range(copies):
+        part = {k: (None if v is None else v[i * len(p):(i + 1) * len(p)]) for k, v in r.items()}
+        H.compare(part, o, p, V, what="floors", check_post=False)
+
+
 def _large_k_rows(oracle, V, seed):
     """Rows with 1024 < top_k < V whose sets end inside buckets of a few, of
     many and of nearly all ids; top-p on, off and near zero."""
