@@ -34,7 +34,7 @@ struct tgs_ctx {
   // one allocation, zeroed once, from k64_lists on
   unsigned long long* k64_lists = nullptr;  // fused kernel chunk lists, [max_batch * kMaxSplit][64]
   unsigned long long* k64_keys = nullptr;   // fused kernel bound-exchange keys, [max_batch][K64_KEYS]
-  unsigned long long* tp_lines = nullptr;   // split top-p exchange lines, [max_batch][TOPPS_LINE]
+  unsigned long long* tp_lines = nullptr;   // split-kernel exchange lines, [max_batch][TOPPS_LINE]
   unsigned* k64_cnt = nullptr;  // fused kernel exchange lines (arrival counter, epoch, count words), one per row
   uint32_t* mask_table = nullptr;
   int n_states = 0, mask_vocab = 0, mask_words = 0;
@@ -216,7 +216,7 @@ struct SampleRes {
   unsigned long long* ws = nullptr;  // [ws_rows][KMAX] general-path chunk lists
   int* ws_cnt = nullptr;             // [ws_rows * (KMAX / 64)]
   int ws_rows = 0;
-  size_t ws_words = 0;                      // ws in 8-byte words (split top-p slabs)
+  size_t ws_words = 0;                      // ws in 8-byte words (split-kernel slabs)
   unsigned long long* tp_lines = nullptr;   // [rows * TOPPS_LINE], zeroed at set-up
   unsigned* k64_cnt = nullptr;              // [rows * K64_CNT_STRIDE], zeroed at set-up
   unsigned long long* k64_lists = nullptr;  // [rows * kMaxSplit][64], entries 0 between calls
@@ -432,7 +432,7 @@ int sample_core(const SampleRes& res, std::string& err, const void* d_logits, tg
 //   [k64 chunk lists: kNaRows * kMaxSplit * 64 u64, entries 0 between calls]
 //   [k64 bound-exchange keys: kNaRows * K64_KEYS u64]
 //   [general-path chunk lists, kNaWsRows * KMAX u64, or split-kernel slabs, kNaSlabs * TOPPS_PAIR u64]
-//   [split top-p exchange lines: kNaRows * TOPPS_LINE u64]
+//   [split-kernel exchange lines: kNaRows * TOPPS_LINE u64]
 //   [k64 exchange lines: kNaRows * K64_CNT_STRIDE u32, counters zero between calls]
 //   [general-path list counts: kNaWsRows * (KMAX / 64) i32]
 // The k64 kernel leaves its lists and counters in that state after every

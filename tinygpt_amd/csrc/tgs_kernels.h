@@ -43,10 +43,9 @@ constexpr int TOPP_NT = 1024;
 constexpr int TOPP_CAP = 2816;
 constexpr int TOPP_MASK_PRE = 2;  // register-resident row vectors requested before the mask words
 
-// Split top-p kernel (rows too long for the top-p kernel's registers):
-// threads per workgroup, chunks per row at most, ids per chunk at most, and
-// in 8-byte words: the exchange line of a row, and of a (row, chunk) its
-// slab (NB masses, NB + 1 counts and a pad), one of the two lists behind it
+// Split kernel (rows over several workgroups): threads per workgroup, chunks
+// per row at most, ids per chunk at most, and in 8-byte words: the exchange
+// line of a row, and of a (row, chunk) its slab (NB masses, NB + 1 counts and a pad), one of the two lists behind it
 // (ids of the cut's and the draw's buckets) and all together.
 constexpr int TOPPS_NT = 512;
 constexpr int TOPPS_MAX_SPLIT = 16;
@@ -94,7 +93,7 @@ struct SampleArgs {
   int full_rows;         // 1: full_kernel runs after the chunk kernels
   int hint_k;            // the launch hint's max_top_k (INT_MAX without a hint)
   int topp_all;          // 1: the top-p kernel alone serves the batch (its greedy rows too)
-  unsigned long long* tp_lines;  // split top-p kernel: [rows][TOPPS_LINE] exchange lines (zero at set-up)
+  unsigned long long* tp_lines;  // split kernel: [rows][TOPPS_LINE] exchange lines (zero at set-up)
   int row0, rows;        // split kernel: the launch's first row (slabs are indexed from it) and its rows
   unsigned div8s, divg;  // and the multipliers that divide by 8 S and by the rows past the last group of 8
   int topp_cap;          // top-p kernel: allowed ids packed into LDS (beyond topp_lds_bytes)
@@ -208,8 +207,9 @@ hipError_t launch_topp(const SampleArgs& a, int dtype, hipStream_t st);
 hipError_t set_topp_lds_limit(size_t bytes);
 // Longest row the top-p kernel holds in registers.
 int topp_resident_ids();
-// The same rows over a.S chunks of a.L ids each, `rows` rows per launch
-// (their slabs lie in a.ws); dynamic LDS topp_lds_bytes.
+// Every kind of row (the top-p kernel's with a.topp_all) over a.S chunks of a.L
+// ids each, at most `rows` rows per launch (their slabs lie in a.ws); dynamic
+// LDS topp_lds_bytes.
 hipError_t launch_topps(SampleArgs a, int dtype, int rows, hipStream_t st);
 size_t topps_static_lds();
 hipError_t set_topps_lds_limit(size_t bytes);

@@ -1,7 +1,8 @@
 // tgs_kernels.hip -- gfx950 kernels of the decode-time sampler.
 //
-// Sampling a [B, V] batch takes one to three launches on the caller's
-// stream:
+// The kernels of the [B, V] batches that no other kernel takes (sample_core in
+// tgs_api.hip: short rows without a hint, and a range of sizes between), in one
+// to three launches on the caller's stream:
 //
 //   chunk_kernel  workgroup (b, c) owns chunk c of row b (S chunks per row).
 //                 It issues all 16-byte loads of its first tile up front,
